@@ -176,12 +176,12 @@ def _f32(*shape):
 
 
 def _t(x):
-    """The ggml descriptor of a torch view: ne[0] is torch's last dimension."""
+    """The ggml descriptor of a torch view: ne[0] is torch's last dimension, and a
+    dimension that x does not have strides over all of x, as in ggml."""
     shape, stride = list(x.shape), list(x.stride())
-    while len(shape) < 4:
-        shape.insert(0, 1)
-        stride.insert(0, shape[1] * stride[1] if len(stride) else 1)
-    return H.tensor(x.data_ptr(), shape[::-1], [4 * s for s in stride[::-1]])
+    lead = 4 - x.dim()
+    span = max(n * s for n, s in zip(shape, stride))
+    return H.tensor(x.data_ptr(), shape[::-1] + [1] * lead, [4 * s for s in stride[::-1]] + [4 * span] * lead)
 
 
 def prepare(case, seed):
