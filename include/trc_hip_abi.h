@@ -142,15 +142,17 @@ int trc_hip_dequant(int type, const void* blocks, int64_t n_blocks, float* dst, 
  * computed by compute_mul_mat (src/backends/cpu/trc_cpu_ops.cpp:182-216).
  * All three tensors are TRC_HIP_TYPE_F32 with 4-byte aligned data and strides.
  * The sum is reordered, so results match the CPU to rounding, not bit for bit;
- * they are the same from run to run. dst must not overlap a or b: for some
- * shapes (K >= 1024, between half and two 128 x 128 output tiles per CU, a
- * contiguous dst) the two halves of the sum over k meet in dst, one stored and
- * the other added, ordered through 32 KiB of ticket words kept past the end of
- * the stream's workspace of trc_hip_qmatvec. The first such call on a stream
- * allocates that workspace (make it before capturing the stream into a graph
- * in global capture mode); the rules for that workspace below hold here too:
- * calls on different streams may overlap, a captured graph keeps the words of
- * the stream it was captured on, and trc_hip_qmatvec_release_stream frees them. */
+ * they are the same from run to run, on every stream and under capture. dst must
+ * not overlap a or b: where few 128 x 128 output tiles leave CUs idle, K is
+ * summed in up to 8 parts that meet in dst or in slots, ordered through 32 KiB of
+ * ticket words kept past the end of the stream's workspace of trc_hip_qmatvec
+ * (the slots, 16 MiB, are an allocation of their own, made by the first call on
+ * the stream that needs them). Where the stream has none and none can be had
+ * without a wait (the stream is being captured, or eight streams hold the
+ * device's workspaces), the parts run one launch after another, with the same
+ * result. The rules for that workspace below hold here too: calls on different
+ * streams may overlap, a captured graph keeps the words and slots of the stream
+ * it was captured on, and trc_hip_qmatvec_release_stream frees them. */
 int trc_hip_mul_mat_f32(const trc_hip_tensor* a, const trc_hip_tensor* b,
                         const trc_hip_tensor* dst, void* stream);
 

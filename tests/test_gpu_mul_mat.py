@@ -440,3 +440,176 @@ def test_mul_mat_acc_rejects_overlap(hip):
     assert e.value.code == H.E_SHAPE
     for t in (buf, b3):
         t.free()
+
+
+# ---------------------------------------------------------------- bf16 tiles (csrc/hip/mm_bf3.h)
+
+def _f64(av, bv):
+    a, b = np.asarray(av, np.float64), np.asarray(bv, np.float64)
+    r3, r2 = b.shape[0] // a.shape[0], b.shape[1] // a.shape[1]
+    return b @ np.swapaxes(np.tile(a, (r3, r2, 1, 1)), 2, 3)
+
+
+def _rel(got, want):
+    return float(np.linalg.norm(got.astype(np.float64) - want) / np.linalg.norm(want))
+
+
+@pytest.mark.parametrize("shape", [
+    # (K, M, N, planes): last slabs of 1, 16, 17 and 31 k and a whole one; parts of K
+    # from 1 to 8; last column tiles of 1, 64, 65 and 128; rows of 1, 3 and 127 past a tile
+    (1025, 257, 129, 1), (2064, 515, 192, 1), (4113, 383, 193, 1), (3103, 129, 70, 1), (2048, 256, 256, 1),
+    (8192, 131, 65, 1), (515, 130, 131, 3), (1056, 128, 128, 8), (160, 1300, 1100, 7),
+])
+@pytest.mark.parametrize("layout", ["kk", "tk", "kt", "tt", "odd", "gen"])
+def test_bf16_tiles_against_float64(hip, shape, layout):
+    """Every element against float64: the 2-norm of the error stays below that of K
+    floats added one after another, sqrt(K) half ulps of the result for normal
+    inputs (2^-25 sqrt(K)). odd: rows 4 bytes off 16-byte alignment; gen: every other
+    element along both dimensions."""
+    K, M, N, P = shape
+    rng = np.random.default_rng(K + M + N)
+    announce(f"mul_mat bf16 tiles {shape} {layout}")
+    if layout == "odd":
+        A, B = (rng.standard_normal((1, P, r, K + 3)).astype(np.float32) for r in (M, N))
+        af = bf = lambda x: x[..., 3:]
+    elif layout == "gen":
+        A, B = (rng.standard_normal((1, P, r, 2 * K)).astype(np.float32) for r in (2 * M, N))
+        af, bf = (lambda x: x[:, :, ::2, ::2]), (lambda x: x[..., ::2])
+    else:
+        ta, tb = layout[0] == "t", layout[1] == "t"
+        A = rng.standard_normal((1, P, K, M) if ta else (1, P, M, K)).astype(np.float32)
+        B = rng.standard_normal((1, P, K, N) if tb else (1, P, N, K)).astype(np.float32)
+        af, bf = (t01 if ta else (lambda x: x)), (t01 if tb else (lambda x: x))
+    da, db = Dev(A), Dev(B)
+    got = gpu_mul_mat(da, af(da.base), db, bf(db.base))
+    da.free()
+    db.free()
+    assert _rel(got, _f64(af(A), bf(B))) <= 2.0 ** -25 * np.sqrt(K)
+
+
+# one shape per way the parts of K come together: K whole on 8-wave and 4-wave
+# workgroups, two parts in dst, more in slots
+BF16_ROUTES = [(640, 1024, 512, 2), (128, 2048, 512, 8), (1024, 2048, 1024, 1), (4096, 512, 200, 1)]
+
+
+@pytest.mark.parametrize("shape", BF16_ROUTES)
+def test_bf16_tiles_special_values(hip, shape):
+    """Infinities, NaNs, values that round to infinity as bf16, subnormals and values
+    whose last bits bf16 cannot hold, each in rows and columns of their own: results
+    are float64's (not finite where it is not, equal to float rounding elsewhere), and
+    the other rows' bits are what they are without them, in tiles that hold none."""
+    K, M, N, P = shape
+    rng = np.random.default_rng(7 * K + M)
+    announce(f"mul_mat bf16 tiles special values {shape}")
+    A = rng.standard_normal((1, P, M, K)).astype(np.float32)
+    B = rng.standard_normal((1, P, N, K)).astype(np.float32)
+    clean = (A.copy(), B.copy())
+    A[0, 0, 3, 5] = np.inf
+    A[0, 0, 4, K - 1] = np.nan
+    A[0, 0, 5] = 0
+    A[0, 0, 5, K // 2] = np.float32(3.4e38)       # infinity as bf16; finite times the column below
+    B[0, 0, :, K // 2] = np.clip(B[0, 0, :, K // 2], -0.9, 0.9)
+    clean[1][0, 0, :, K // 2] = B[0, 0, :, K // 2]
+    A[0, 0, 6] = (rng.standard_normal(K) * 1e-38).astype(np.float32)
+    A[0, 0, 7] = (rng.standard_normal(K) * 1e-41).astype(np.float32)
+    B[0, 0, 2] *= np.float32(1e20)
+    clean[1][0, 0, 2] = B[0, 0, 2]
+    B[0, 0, 9, 0] = -np.inf
+    clean[1][0, 0, 9] = B[0, 0, 9]
+    da, db, dc = Dev(A), Dev(B), Dev(clean[0])
+    got = gpu_mul_mat(da, A, db, B)
+    plain = gpu_mul_mat(dc, clean[0], db, B)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = _f64(A[:, :1], B[:, :1])[0, 0]     # [N, M]
+        w32 = want.astype(np.float32)
+    g = got[0, 0]
+    assert np.array_equal(np.isnan(g), np.isnan(w32))
+    assert np.array_equal(g[np.isinf(w32)], w32[np.isinf(w32)])
+    ok = np.isfinite(w32)
+    a, b = (np.abs(np.nan_to_num(x[0, 0], posinf=0, neginf=0).astype(np.float64)) for x in (A, B))
+    scale = b @ a.T
+    # K additions of half an ulp each, and half the smallest subnormal for each
+    bound = K * (2.0 ** -24 * scale + 2.0 ** -150)
+    assert np.all(np.abs(g[ok].astype(np.float64) - want[ok]) <= bound[ok])
+    # beyond the first tiles' rows nothing has changed
+    assert np.array_equal(got[:, :, :, 128:].view(np.uint32), plain[:, :, :, 128:].view(np.uint32))
+    for d in (da, db, dc):
+        d.free()
+
+
+@pytest.mark.parametrize("shape", BF16_ROUTES)
+def test_bf16_tiles_integers_are_exact(hip, shape):
+    """Integer operands whose sums stay under 2^24: every sum is exact in float, so
+    the bits are those of any order of adding."""
+    K, M, N, P = shape
+    rng = np.random.default_rng(K)
+    announce(f"mul_mat bf16 tiles integers {shape}")
+    A = rng.integers(-60, 61, (1, P, M, K)).astype(np.float32)
+    B = rng.integers(-60, 61, (1, P, N, K)).astype(np.float32)
+    A[0, 0, 0], B[0, 0, 0] = 0, 0
+    A[0, 0, 0, K // 3], B[0, 0, 0, K // 3] = 1, 16777215.0
+    da, db = Dev(A), Dev(B)
+    got = gpu_mul_mat(da, A, db, B)
+    da.free()
+    db.free()
+    want = _f64(A, B)
+    small = np.abs(want) < 2 ** 24
+    small[0, 0, 0, 1:] = False                    # that column's other sums pass 2^24
+    assert small.mean() > 0.99
+    assert np.array_equal(got[small], want[small].astype(np.float32))
+
+
+def test_bf16_tiles_without_a_workspace(hip):
+    """Where a stream has no workspace and none may be made (eight other streams hold
+    the device's, or the stream is under capture), the parts of K run one launch
+    after another: the same bits as when they meet."""
+    import ctypes as C
+
+    from gpu_util import runtime
+    rt = runtime()
+    announce("mul_mat bf16 tiles, nine streams and capture")
+    cases = []
+    for K, M, N in [(2048, 512, 200), (1024, 2048, 1024)]:
+        A, B = synth.normal(960 + M, K * M).reshape(1, 1, M, K), synth.normal(961 + N, K * N).reshape(1, 1, N, K)
+        cases.append((Dev(A), Dev(B), empty((1, 1, N, M))))
+    H.qmatvec_release_stream(None)
+    live = [Stream() for _ in range(10)]
+    refs = []
+    for s in live:
+        for c, (a, b, d) in enumerate(cases):
+            H.mul_mat_f32(a.tensor(), b.tensor(), d.tensor(), s.handle)
+            H.sync(s.handle)
+            got = d.read().copy()
+            if len(refs) <= c:
+                refs.append(got)
+                assert _rel(got, _f64(a.base, b.base)) <= 2.0 ** -25 * np.sqrt(a.base.shape[3])
+            assert np.array_equal(got.view(np.uint32), refs[c].view(np.uint32))
+    for s in live:
+        s.close()
+    s = Stream()
+    graph, gexec = C.c_void_p(), C.c_void_p()
+    assert rt.hipStreamBeginCapture(C.c_void_p(s.handle), 0) == 0
+    try:
+        for a, b, d in cases:
+            H.mul_mat_f32(a.tensor(), b.tensor(), d.tensor(), s.handle)
+    finally:
+        rc = rt.hipStreamEndCapture(C.c_void_p(s.handle), C.byref(graph))
+    assert rc == 0
+    assert rt.hipGraphInstantiate(C.byref(gexec), graph, None, None, 0) == 0
+    for _ in range(3):
+        for a, b, d in cases:
+            H.fill_f32(d.ptr, float("nan"), d.base.size)
+        H.sync()
+        assert rt.hipGraphLaunch(gexec, C.c_void_p(s.handle)) == 0
+        H.sync(s.handle)
+        for (a, b, d), ref in zip(cases, refs):
+            assert np.array_equal(d.read().view(np.uint32), ref.view(np.uint32))
+            H.mul_mat_f32(a.tensor(), b.tensor(), d.tensor(), s.handle)  # eager, between the replays
+            H.sync(s.handle)
+            assert np.array_equal(d.read().view(np.uint32), ref.view(np.uint32))
+    rt.hipGraphExecDestroy(gexec)
+    rt.hipGraphDestroy(graph)
+    s.close()
+    for a, b, d in cases:
+        for x in (a, b, d):
+            x.free()

@@ -74,6 +74,29 @@ __device__ __forceinline__ void ticket_clear(uint32_t* tk, int lane) {
     }
 }
 
+// More than two parts, their sums in slots of a workspace: every part but the
+// last to take a ticket stores its sums (device scope), waits for the stores and
+// counts itself in tk[1]; the last waits for that count, which no part that has
+// its ticket holds up, and reads the slots.
+__device__ __forceinline__ bool ticket_last(uint32_t* tk, int lane, uint32_t parts) {
+    uint32_t n = 0;
+    if (lane == 0) n = __hip_atomic_fetch_add(tk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_amdgcn_readfirstlane(n) == parts - 1;
+}
+__device__ __forceinline__ void ticket_arrive(uint32_t* tk, int lane) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (lane == 0) (void) __hip_atomic_fetch_add(tk + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void ticket_wait_all(uint32_t* tk, int lane, uint32_t others) {
+    if (lane == 0) {
+        for (int n = 0; n < TICKET_FLAG_POLLS; ++n) {
+            if (__hip_atomic_load(tk + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == others) break;
+            __builtin_amdgcn_s_sleep(1);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // Launch-side error reporting, implemented in abi.hip.
 int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);
@@ -114,7 +137,12 @@ int qm_release_stream(hipStream_t stream);
 // MM_TICKETS of them), kept past the end of the stream's workspace: zero when
 // the workspace is made, and left zero by every launch that uses them.
 constexpr int MM_TICKETS = 512 * 8 * 2;
-int mm_stream_tickets(hipStream_t stream, uint32_t** tickets);
+// mm_stream_scratch: these words, and where `slots` is not 0 that many 64 KiB slots (at most
+// MM_SLOTS) for the sums of K's parts, or null for both where there are none to
+// be had without a wait: the stream has no workspace yet and it is being
+// captured, or as many streams as the device keeps workspaces for have one.
+constexpr size_t MM_SLOTS = 256;
+int mm_stream_scratch(hipStream_t stream, size_t slots, uint32_t** tickets, float** sums);
 int launch_add_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const trc_hip_tensor& d, hipStream_t stream);
 int launch_mul_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const trc_hip_tensor& d, hipStream_t stream);
 int launch_repeat_f32(const trc_hip_tensor& a, const trc_hip_tensor& d, hipStream_t stream);

@@ -1,0 +1,77 @@
+// The bf16 tile kernel (mm_bf3.h) with K whole, and the choice and launch of its
+// tiles. The parts of K that meet are in mm_bf3_parts.hip.
+#include "mm_bf3.h"
+
+namespace trc_hip {
+
+int launch_mm_bf3_pair(const MMArgs& p, unsigned grid, hipStream_t s);
+int launch_mm_bf3_slots(const MMArgs& p, unsigned grid, hipStream_t s);
+
+bool mm_bf3_fits(const MMArgs& p) {
+    // 32-bit buffer offsets over the rows of a tile
+    auto span = [](int64_t n0, int64_t nb0, int64_t n1, int64_t nb1) { return (n0 - 1) * nb0 + (n1 - 1) * nb1 + 4; };
+    const int64_t ti = p.M < B3_T ? p.M : B3_T, tj = p.N < B3_T ? p.N : B3_T;
+    return span(p.K, p.a_nb0, ti, p.a_nb1) <= MM_PAST && span(p.K, p.b_nb0, tj, p.b_nb1) <= MM_PAST &&
+           span(ti, p.d_nb0, tj, p.d_nb1) <= MM_PAST;
+}
+
+B3Plan mm_bf3_plan(const MMArgs& p, int64_t planes, int max_parts) {
+    // Times in us, measured where one workgroup of 8 waves has a CU: a 32-deep
+    // slab 0.8, a launch with K whole 7.5 (6.4 to 9, K = 130 to 4096), with K in parts 8 +
+    // 1.6 per part (16 to 64 tiles; two parts that meet in dst 12, six 17, eight
+    // 19 to 24). 4096 x 4096 x 128, parts 1, 2, 3, 4, 6, 8: 107.6, 63.0, 45.5,
+    // 38.9, 34.9, 39.2; 1024 x 1024 x 512: 32.3, 25.1, 20.6, 20.9, 21.9, 27.2.
+    const int64_t tiles = ((p.M + B3_T - 1) / B3_T) * ((p.N + B3_T - 1) / B3_T) * planes;
+    const int64_t cus = device_cus();
+    const double slabs = (double) ((p.K + 31) / 32);
+    const double slab = p.N <= 64 ? 0.7 : 0.8;
+    B3Plan best{2, 1, 7.5 + slab * slabs * (double) ((tiles + cus - 1) / cus)};
+    for (int parts = 2; parts <= max_parts; ++parts) {
+        // a part is at least 4 slabs: shorter ones are all launch and meeting
+        if (slabs < 4 * parts || tiles * parts > (parts == 2 ? 4 * cus : cus)) break;
+        if (parts > 2 && tiles * parts > (int64_t) MM_SLOTS) break;
+        if (tiles * 16 > MM_TICKETS) break;
+        const double each = (double) (((int64_t) slabs + parts - 1) / parts);
+        const double us = 8 + 1.6 * parts + slab * each * (double) ((tiles * parts + cus - 1) / cus);
+        if (us < best.us) best = {2, parts, us};
+    }
+    // More tiles than CUs with K whole: 4-wave workgroups, two to a CU, whose
+    // prologues and stores overlap the other's MFMAs (4096 x 4096 x 512 99 ->
+    // 90 us, configuration 4 143 -> 106 us).
+    if (best.parts == 1 && tiles > cus) best.groups = 1;
+    return best;
+}
+
+int launch_mm_bf3(MMArgs& p, int64_t planes, int groups, int parts, bool acc, hipStream_t s) {
+    p.tiles_i = (p.M + B3_T - 1) / B3_T;
+    p.tiles_j = (p.N + B3_T - 1) / B3_T;
+    p.xcd_planes = planes % 8 == 0 ? 1 : 0;
+    const int64_t tiles = p.tiles_i * p.tiles_j * planes;
+    if (tiles * parts > 0x7FFFFFFF) {
+        return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) tiles * parts);
+    }
+    const unsigned n = (unsigned) tiles;
+    // parts of whole slabs, none of them empty
+    const int64_t slabs = (p.K + 16 * groups - 1) / (16 * groups), per = (slabs + parts - 1) / parts;
+    p.parts = (uint32_t) ((slabs + per - 1) / per);
+    p.part = 0;
+    if (p.parts > 1) {
+        float* slots = nullptr;
+        const bool pair = p.parts == 2;
+        const int rc = mm_stream_scratch(s, pair ? 0 : (size_t) tiles * p.parts, &p.tickets, &slots);
+        if (rc != TRC_HIP_OK) return rc;
+        p.slots = slots;
+        if (p.tickets != nullptr && pair) return launch_mm_bf3_pair(p, n * 2, s);
+        if (p.tickets != nullptr) return launch_mm_bf3_slots(p, n * p.parts, s);
+        // no workspace to meet in: one launch after another, each part added to dst
+        for (; p.part < (int) p.parts; ++p.part) {
+            const int lrc = p.part == 0 ? b3_launch<2, B3_ALONE, false>(p, n, s) : b3_launch<2, B3_ALONE, true>(p, n, s);
+            if (lrc != TRC_HIP_OK) return lrc;
+        }
+        return TRC_HIP_OK;
+    }
+    if (acc) return groups == 2 ? b3_launch<2, B3_ALONE, true>(p, n, s) : b3_launch<1, B3_ALONE, true>(p, n, s);
+    return groups == 2 ? b3_launch<2, B3_ALONE, false>(p, n, s) : b3_launch<1, B3_ALONE, false>(p, n, s);
+}
+
+}  // namespace trc_hip

@@ -1,4 +1,5 @@
-// H3: ggml-semantics F32 mul_mat on the gfx950 FP32 matrix cores.
+// H3: ggml-semantics F32 mul_mat on the gfx950 matrix cores: the FP32 tiles, the
+// few-column kernel, and the choice between them and the bf16 tiles.
 //
 //   dst[i,j,i2,i3] = sum_k a[k,i,i2%a2,i3%a3] * b[k,j,i2,i3]
 //
@@ -31,42 +32,21 @@
 //     put on XCD p % 8, so each src1 plane (and, under the modulo broadcast,
 //     each src0 plane) is read into one L2 only; otherwise tiles follow the
 //     grid order, where the tiles sharing one src0 row block meet on one XCD.
-//   - When 128x128 tiles would give under two workgroups per CU, K is split in
-//     two: 8-wave workgroups (64x32 per wave) each sum half of K for one tile.
-//     The two waves that hold one 64x32 block meet in dst without a clear: each
-//     takes a ticket; the first stores its sums, the second adds its own with
-//     float atomics once the first's are in. a + b is the same in either order,
-//     so results stay deterministic. With whole tiles and float4 loaders the
-//     split products take k_mul_mat_db: two LDS slab buffers, the stores and
-//     loads of the next slabs spread between the MFMAs, one barrier per slab.
+//   - Larger products run on the bf16 matrix cores instead, each float held
+//     exactly as three bf16 (mm_bf3.h): launch_mul_mat_f32 weighs the two. What
+//     stays here are products too small for those tiles and operands whose tiles
+//     span 2 GiB.
 //   - Up to 64 columns against a k-contiguous src0 (decode-sized batches) take
 //     k_mm_skinny below instead: one pass over src0 on every CU.
 #include "common.h"
+#include "mm_args.h"
 
-#include <type_traits>
 
 namespace trc_hip {
 namespace {
 
 
-enum LoadMode { K_CONTIG = 0, R_CONTIG = 1, GENERIC = 2 };
-
-struct MMArgs {
-    const uint8_t* a;
-    const uint8_t* b;
-    uint8_t* d;
-    int64_t K, M, N;
-    int64_t a_nb0, a_nb1, a_nb2, a_nb3, a_ne2, a_ne3;
-    int64_t b_nb0, b_nb1, b_nb2, b_nb3, b_ne2;
-    int64_t d_nb0, d_nb1, d_nb2, d_nb3;
-    int64_t tiles_i, tiles_j;
-    int xcd_planes;  // 1: planes % 8 == 0, tiles of plane p on XCD p % 8
-    int64_t d_span;  // bytes from a dst plane's first element to past its last
-    uint32_t* tickets;  // K split in two: two words per wave of every tile, zero between launches
-};
-
-constexpr uint32_t MM_RSRC_WORD3 = 0x00020000u;  // gfx9 buffer resource: raw 32-bit dwords
-constexpr uint32_t MM_OUT = 0x80000000u;         // an offset past the resource: loads read 0, stores drop
+constexpr int K_CONTIG = MM_K_CONTIG, R_CONTIG = MM_R_CONTIG, GENERIC = MM_GENERIC;
 
 // Loads a ROWS x BK slab (rows = i for src0, j for src1) of one operand into
 // registers, then stores it to LDS as lds[k * LD + row]. The k-contiguous
@@ -78,10 +58,7 @@ constexpr uint32_t MM_OUT = 0x80000000u;         // an offset past the resource:
 // pitch of ROWS + 4, 20 % of the forward product's LDS cycles were
 // bank-conflict stalls, and 4-way conflicts made 128 x 64 tiles at BK = 32 11 %
 // slower.) The other loaders store float4s, whose rows stay 16-byte aligned.
-// KI (k-contiguous only): the slab is stored as planes of k pairs, element
-// (k, row) at (k / 2) * 2 * LD + 2 * row + k % 2, so one 8-byte read gives a
-// lane the two k of a row that two consecutive MFMAs take from it.
-template <int MODE, int ROWS, int BK, int THREADS, bool KI = false>
+template <int MODE, int ROWS, int BK, int THREADS>
 struct SlabLoader {
     static_assert(MODE != K_CONTIG || BK % 16 == 0, "k-contiguous slabs come in 16-k groups");
     static constexpr int LD = MODE == K_CONTIG ? ROWS + 2 : ROWS + 4;
@@ -143,13 +120,8 @@ struct SlabLoader {
                 const int q = tid + THREADS * u;
                 const int row = (q >> 2) % ROWS;
                 const int kq = (q & 3) + 4 * (q / (4 * ROWS));
-                if constexpr (KI) {
-                    *(float2*) (lds + (2 * kq) * 2 * LD + 2 * row) = float2{r[4 * u + 0], r[4 * u + 1]};
-                    *(float2*) (lds + (2 * kq + 1) * 2 * LD + 2 * row) = float2{r[4 * u + 2], r[4 * u + 3]};
-                } else {
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) lds[(4 * kq + c) * LD + row] = r[4 * u + c];
-                }
+                for (int c = 0; c < 4; ++c) lds[(4 * kq + c) * LD + row] = r[4 * u + c];
             }
         } else if constexpr (MODE == R_CONTIG) {
 #pragma unroll
@@ -170,17 +142,14 @@ struct SlabLoader {
     }
 };
 
-// SPLIT: parts of K (1, or 2 meeting in dst through the stream's ticket words).
-// ACC: dst += the product (K in one part).
-template <int WI, int WJ, int TI, int TJ, int BK, int AMODE, int BMODE, int SPLIT, bool ACC = false, bool KI = false>
+// ACC: dst += the product.
+template <int WI, int WJ, int TI, int TJ, int BK, int AMODE, int BMODE, bool ACC = false>
 __global__ __launch_bounds__(WI * WJ * 64) void k_mul_mat(MMArgs p) {
     constexpr int THREADS = WI * WJ * 64;
-    static_assert(SPLIT == 1 || SPLIT == 2, "two parts at most keep the atomic sums deterministic");
-    static_assert(!ACC || SPLIT == 1, "d + a + b would round differently from d + (a + b)");
     constexpr int BM = WI * TI * 32;  // tile extent along i
     constexpr int BN = WJ * TJ * 32;  // tile extent along j
-    using LA = SlabLoader<AMODE, BM, BK, THREADS, KI && AMODE == K_CONTIG>;
-    using LB = SlabLoader<BMODE, BN, BK, THREADS, KI && BMODE == K_CONTIG>;
+    using LA = SlabLoader<AMODE, BM, BK, THREADS>;
+    using LB = SlabLoader<BMODE, BN, BK, THREADS>;
     __shared__ __attribute__((aligned(16))) float As[BK * LA::LD];
     __shared__ __attribute__((aligned(16))) float Bs[BK * LB::LD];
 
@@ -193,12 +162,9 @@ __global__ __launch_bounds__(WI * WJ * 64) void k_mul_mat(MMArgs p) {
     int64_t t = blockIdx.x;
     if (p.xcd_planes) {
         // workgroup b = 8k + x runs on XCD x: give it tile k % tpp of plane 8 (k / tpp) + x
-        const int64_t tpp = p.tiles_i * p.tiles_j * SPLIT, x = t & 7, k = t >> 3;
+        const int64_t tpp = p.tiles_i * p.tiles_j, x = t & 7, k = t >> 3;
         t = (8 * (k / tpp) + x) * tpp + k % tpp;
     }
-    const int part = SPLIT > 1 ? (int) (t % SPLIT) : 0;
-    t /= SPLIT;
-    const int64_t tile = t;
     const int64_t ti = t % p.tiles_i;
     t /= p.tiles_i;
     const int64_t tj = t % p.tiles_j;
@@ -222,13 +188,9 @@ __global__ __launch_bounds__(WI * WJ * 64) void k_mul_mat(MMArgs p) {
 
     LA la;
     LB lb;
-    // this part's slabs: [kt0, kt0 + nk)
-    const int64_t slabs = (p.K + BK - 1) / BK;
-    const int64_t per_part = (slabs + SPLIT - 1) / SPLIT;
-    const int64_t kt0 = part * per_part;
-    const int64_t nk = slabs - kt0 < per_part ? slabs - kt0 : per_part;
-    la.load(a, p.a_nb0, p.a_nb1, i0, p.M, kt0 * BK, p.K, tid);
-    lb.load(b, p.b_nb0, p.b_nb1, j0, p.N, kt0 * BK, p.K, tid);
+    const int64_t nk = (p.K + BK - 1) / BK;
+    la.load(a, p.a_nb0, p.a_nb1, i0, p.M, 0, p.K, tid);
+    lb.load(b, p.b_nb0, p.b_nb1, j0, p.N, 0, p.K, tid);
     la.store(As, tid);
     lb.store(Bs, tid);
     __syncthreads();
@@ -238,64 +200,28 @@ __global__ __launch_bounds__(WI * WJ * 64) void k_mul_mat(MMArgs p) {
     for (int64_t kt = 0; kt < nk; ++kt) {
         const bool more = kt + 1 < nk;
         if (more) {
-            la.load(a, p.a_nb0, p.a_nb1, i0, p.M, (kt0 + kt + 1) * BK, p.K, tid);
-            lb.load(b, p.b_nb0, p.b_nb1, j0, p.N, (kt0 + kt + 1) * BK, p.K, tid);
+            la.load(a, p.a_nb0, p.a_nb1, i0, p.M, (kt + 1) * BK, p.K, tid);
+            lb.load(b, p.b_nb0, p.b_nb1, j0, p.N, (kt + 1) * BK, p.K, tid);
         }
-        // Several 4-wave workgroups share a CU without a K split: a wave in its
-        // MFMA block issues ahead of the others' loads, stores and barriers
-        // (dW 142 -> 136 us, configuration 4 168 -> 161 us, same bits). The split
-        // products run one workgroup per CU, where it measured no gain.
-        if constexpr (SPLIT == 1) __builtin_amdgcn_s_setprio(1);
-        if constexpr (KI) {
-            // k in groups of 4: the first MFMA of a group takes k = 4t + 2 half, the
-            // second 4t + 2 half + 1, from both operands
+        // Several 4-wave workgroups share a CU: a wave in its MFMA block issues
+        // ahead of the others' loads, stores and barriers (128 x 128 tiles at K =
+        // 512: 142 -> 136 us, same bits).
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int t4 = 0; t4 < BK / 4; ++t4) {
-                const int k0 = 4 * t4 + 2 * half;
-                float2 av[TI], bv[TJ];
+        for (int s = 0; s < BK / 2; ++s) {
+            const int kr = 2 * s + half;
+            float av[TI], bv[TJ];
 #pragma unroll
-                for (int x = 0; x < TI; ++x) {
-                    const int r = (wi * TI + x) * 32 + col;
-                    if constexpr (AMODE == K_CONTIG) {
-                        av[x] = *(const float2*) (As + (k0 >> 1) * 2 * LA::LD + 2 * r);
-                    } else {
-                        av[x] = float2{As[k0 * LA::LD + r], As[(k0 + 1) * LA::LD + r]};
-                    }
-                }
+            for (int x = 0; x < TI; ++x) av[x] = As[kr * LA::LD + (wi * TI + x) * 32 + col];
 #pragma unroll
-                for (int y = 0; y < TJ; ++y) {
-                    const int r = (wj * TJ + y) * 32 + col;
-                    if constexpr (BMODE == K_CONTIG) {
-                        bv[y] = *(const float2*) (Bs + (k0 >> 1) * 2 * LB::LD + 2 * r);
-                    } else {
-                        bv[y] = float2{Bs[k0 * LB::LD + r], Bs[(k0 + 1) * LB::LD + r]};
-                    }
-                }
+            for (int y = 0; y < TJ; ++y) bv[y] = Bs[kr * LB::LD + (wj * TJ + y) * 32 + col];
 #pragma unroll
-                for (int x = 0; x < TI; ++x)
+            for (int x = 0; x < TI; ++x)
 #pragma unroll
-                    for (int y = 0; y < TJ; ++y) {
-                        acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[y].x, av[x].x, acc[x][y], 0, 0, 0);
-                        acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[y].y, av[x].y, acc[x][y], 0, 0, 0);
-                    }
-            }
-        } else {
-#pragma unroll
-            for (int s = 0; s < BK / 2; ++s) {
-                const int kr = 2 * s + half;
-                float av[TI], bv[TJ];
-#pragma unroll
-                for (int x = 0; x < TI; ++x) av[x] = As[kr * LA::LD + (wi * TI + x) * 32 + col];
-#pragma unroll
-                for (int y = 0; y < TJ; ++y) bv[y] = Bs[kr * LB::LD + (wj * TJ + y) * 32 + col];
-#pragma unroll
-                for (int x = 0; x < TI; ++x)
-#pragma unroll
-                    for (int y = 0; y < TJ; ++y)
-                        acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[y], av[x], acc[x][y], 0, 0, 0);
-            }
+                for (int y = 0; y < TJ; ++y)
+                    acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[y], av[x], acc[x][y], 0, 0, 0);
         }
-        if constexpr (SPLIT == 1) __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_s_setprio(0);
         if (more) {
             __syncthreads();
             la.store(As, tid);
@@ -361,44 +287,6 @@ __global__ __launch_bounds__(WI * WJ * 64) void k_mul_mat(MMArgs p) {
         }
         return;
     }
-    if constexpr (SPLIT > 1) {
-        // dst element of accumulator register v of tile (x, y), or null past dst
-        auto out = [&](int x, int y, int v) -> float* {
-            const int64_t i = i0 + (wi * TI + x) * 32 + col;
-            const int64_t j = j0 + (wj * TJ + y) * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
-            return i < p.M && j < p.N ? (float*) (d + i * p.d_nb0 + j * p.d_nb1) : nullptr;
-        };
-        // The waves holding this 64 x 32 block in the two parts meet through two
-        // ticket words (ticket_first and the protocol it begins, common.h).
-        // Against a cleared dst with an atomic add from each part, this leaves
-        // out the clearing launch and half of the atomics (configuration 3's
-        // forward and dX products 156.7 -> 150.5 and 155.6 -> 149.4 us), with
-        // the same sums.
-        uint32_t* tk = p.tickets + 2 * (tile * (WI * WJ) + wave);
-        if (ticket_first(tk, lane)) {
-#pragma unroll
-            for (int x = 0; x < TI; ++x)
-#pragma unroll
-                for (int y = 0; y < TJ; ++y)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v)
-                        if (float* o = out(x, y, v))
-                            __hip_atomic_store(o, acc[x][y][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            ticket_publish(tk, lane);
-            return;
-        }
-        ticket_wait(tk, lane);
-#pragma unroll
-        for (int x = 0; x < TI; ++x)
-#pragma unroll
-            for (int y = 0; y < TJ; ++y)
-#pragma unroll
-                for (int v = 0; v < 16; ++v)
-                    if (float* o = out(x, y, v))
-                        __hip_atomic_fetch_add(o, acc[x][y][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ticket_clear(tk, lane);
-        return;
-    }
 #pragma unroll
     for (int x = 0; x < TI; ++x) {
         const int64_t i = i0 + (wi * TI + x) * 32 + col;
@@ -415,309 +303,6 @@ __global__ __launch_bounds__(WI * WJ * 64) void k_mul_mat(MMArgs p) {
             }
         }
     }
-}
-
-// ------------------------------------------ double-buffered slabs, whole tiles
-//
-// 128 x 128 tiles on 8-wave workgroups (64 x 32 per wave) when every tile and
-// slab is whole (M and N multiples of 128, K of 2 slabs per part) and both
-// operands load as float4s (k- or row-contiguous). k_mul_mat stores each slab
-// between two barriers while no MFMA runs, with both waves of every SIMD
-// waiting together; here two LDS slab buffers take turns: during the MFMAs of
-// slab s the registers holding slab s + 1 are stored into the idle buffer (one
-// float4 piece per group of 4 k, from group S0 on) and then refilled with slab
-// s + 2 (from group L0 on), with one barrier per slab. Whole tiles need no
-// bounds checks, which keeps the slab loop free of branches and selects (with
-// clamped addresses and selects the split schedule measured 157-160 us, slower
-// than k_mul_mat). Both operands are read as k-paired LDS planes where they are
-// k-contiguous, so the MFMAs take k in groups of 4 (k = 4t + 2 half, then
-// 4t + 2 half + 1). Two uses (interleaved minimums, one box, configuration 3 /
-// 4):
-//   - K split in two (DbPlan<2, ...>: 32-deep slabs, default priority), the
-//     parts meeting in dst through the stream's ticket words as in k_mul_mat:
-//     forward 149.5 -> 137.4 us (its sums now group k by pairs, within 6e-5 of
-//     281), dX 148.8 -> 146.0 us (same bits);
-//   - K whole (DbPlan<1, ...>: 16-deep slabs, two workgroups per CU, the MFMA-block
-//     priority of k_mul_mat): dW 135.3 -> 129.7 us, configuration 4 158.5 ->
-//     147.2 us; ACC adds the product into dst as k_mul_mat's ACC does.
-constexpr int DB_WI = 2, DB_WJ = 4, DB_TI = 2, DB_TJ = 1;
-constexpr int DB_THREADS = DB_WI * DB_WJ * 64;
-constexpr int DB_BM = DB_WI * DB_TI * 32, DB_BN = DB_WJ * DB_TJ * 32;
-// slab depth, the group of 4 k from which a slab's pieces are stored (S0) and
-// the next slab's loaded (L0), and the MFMA-block priority, per number of K
-// parts and src0 layout. Measured on configuration 3 (µs): the forward product
-// (k-contiguous src0) 140.0 with S0 = 1, 137.3-137.5 with S0 = 0 and L0 = 1..4;
-// dX (row-contiguous src0) 146.0-146.2 with S0 = 1 and L0 = 3..4, 146.9-149.9
-// with S0 = 0 or 2; the priority made both slower (141.0, 153.3), 64-deep slabs
-// changed them by under 1 %.
-template <int SPLIT, int AMODE>
-struct DbPlan;
-template <int AMODE>
-struct DbPlan<2, AMODE> {
-    static constexpr int BK = 32, S0 = AMODE == K_CONTIG ? 0 : 1, L0 = AMODE == K_CONTIG ? 2 : 4;
-    static constexpr bool PRIO = false;
-};
-template <int AMODE>
-struct DbPlan<1, AMODE> {
-    static constexpr int BK = 16, S0 = 0, L0 = 1;
-    static constexpr bool PRIO = true;
-};
-
-// One operand's slab as NU float4 pieces per thread: the K_CONTIG mapping of
-// SlabLoader (4 lanes per 64 contiguous bytes of a row, then rows, then k) with
-// k-paired planes, or the R_CONTIG one (float4s along the rows of one k).
-template <int MODE, int ROWS, int BK>
-struct SlabPieces {
-    static_assert(MODE != K_CONTIG || BK % 16 == 0, "k-contiguous pieces come in 16-k groups");
-    static_assert(ROWS * BK % (DB_THREADS * 4) == 0, "whole float4 pieces per thread");
-    static constexpr int LD = MODE == K_CONTIG ? ROWS + 2 : ROWS + 4;
-    static constexpr int NU = ROWS * BK / DB_THREADS / 4;
-    static constexpr int SZ = BK * LD;
-    const uint8_t* src[NU];  // piece u of the part's first slab
-    int lo[NU];              // its LDS float offset
-    int64_t step;            // bytes from one slab to the next
-    f4 r[NU];
-
-    __device__ __forceinline__ void init(const uint8_t* base, int64_t nb_k, int64_t nb_r, int64_t row0, int64_t k0,
-                                         int tid) {
-#pragma unroll
-        for (int u = 0; u < NU; ++u) {
-            const int q = tid + DB_THREADS * u;
-            if constexpr (MODE == K_CONTIG) {
-                const int row = (q >> 2) % ROWS, kq = (q & 3) + 4 * (q / (4 * ROWS));
-                src[u] = base + (row0 + row) * nb_r + (k0 + 4 * kq) * 4;
-                lo[u] = (2 * kq) * 2 * LD + 2 * row;
-            } else {
-                const int k = q / (ROWS / 4), rq = q % (ROWS / 4);
-                src[u] = base + (row0 + 4 * rq) * 4 + (k0 + k) * nb_k;
-                lo[u] = k * LD + 4 * rq;
-            }
-        }
-        step = MODE == K_CONTIG ? (int64_t) BK * 4 : (int64_t) BK * nb_k;
-    }
-    __device__ __forceinline__ void load(int64_t s, int u) { r[u] = *(const f4*) (src[u] + s * step); }
-    __device__ __forceinline__ void store(float* l, int u) const {
-        if constexpr (MODE == K_CONTIG) {
-            *(float2*) (l + lo[u]) = float2{r[u].x, r[u].y};
-            *(float2*) (l + lo[u] + 2 * LD) = float2{r[u].z, r[u].w};
-        } else {
-            *(f4*) (l + lo[u]) = r[u];
-        }
-    }
-    // the k pair (k0, k0 + 1) of row r, k0 even
-    __device__ __forceinline__ static float2 pair(const float* l, int k0, int r) {
-        if constexpr (MODE == K_CONTIG) return *(const float2*) (l + (k0 >> 1) * 2 * LD + 2 * r);
-        else return float2{l[k0 * LD + r], l[(k0 + 1) * LD + r]};
-    }
-};
-
-template <int AMODE, int BMODE, int SPLIT, bool ACC = false>
-__global__ __launch_bounds__(DB_THREADS) void k_mul_mat_db(MMArgs p) {
-    using PL = DbPlan<SPLIT, AMODE>;
-    constexpr int BK = PL::BK;
-    using PA = SlabPieces<AMODE, DB_BM, BK>;
-    using PB = SlabPieces<BMODE, DB_BN, BK>;
-    constexpr int NU = PA::NU + PB::NU;
-    static_assert(!ACC || SPLIT == 1, "d + a + b would round differently from d + (a + b)");
-    static_assert(PL::L0 >= PL::S0, "a piece's registers are stored before the load of the slab after refills them");
-    static_assert(PL::S0 + NU <= BK / 4 && PL::L0 + NU <= BK / 4, "every piece is placed within the slab's k groups");
-    __shared__ __attribute__((aligned(16))) float As[2][PA::SZ];
-    __shared__ __attribute__((aligned(16))) float Bs[2][PB::SZ];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wi = wave % DB_WI, wj = wave / DB_WI;
-    const int half = lane >> 5, col = lane & 31;
-
-    int64_t t = blockIdx.x;
-    if (p.xcd_planes) {
-        const int64_t tpp = p.tiles_i * p.tiles_j * SPLIT, x = t & 7, k = t >> 3;
-        t = (8 * (k / tpp) + x) * tpp + k % tpp;
-    }
-    const int part = SPLIT > 1 ? (int) (t % SPLIT) : 0;
-    t /= SPLIT;
-    const int64_t tile = t;
-    const int64_t ti = t % p.tiles_i;
-    t /= p.tiles_i;
-    const int64_t tj = t % p.tiles_j;
-    const int64_t plane = t / p.tiles_j;
-    const int64_t i2 = plane % p.b_ne2, i3 = plane / p.b_ne2;
-    const uint8_t* a = p.a + (i2 % p.a_ne2) * p.a_nb2 + (i3 % p.a_ne3) * p.a_nb3;
-    const uint8_t* b = p.b + i2 * p.b_nb2 + i3 * p.b_nb3;
-    uint8_t* d = p.d + i2 * p.d_nb2 + i3 * p.d_nb3;
-    const int64_t i0 = ti * DB_BM, j0 = tj * DB_BN;
-    const int64_t nk = p.K / BK / SPLIT;  // slabs per part (at least 2)
-    PA pa;
-    PB pb;
-    pa.init(a, p.a_nb0, p.a_nb1, i0, part * nk * BK, tid);
-    pb.init(b, p.b_nb0, p.b_nb1, j0, part * nk * BK, tid);
-    auto gload = [&](int64_t s, int u) {
-        if (u < PA::NU) pa.load(s, u);
-        else pb.load(s, u - PA::NU);
-    };
-    auto lstore = [&](int buf, int u) {
-        if (u < PA::NU) pa.store(As[buf], u);
-        else pb.store(Bs[buf], u - PA::NU);
-    };
-
-    f16v acc[DB_TI][DB_TJ];
-#pragma unroll
-    for (int x = 0; x < DB_TI; ++x)
-#pragma unroll
-        for (int y = 0; y < DB_TJ; ++y)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[x][y][v] = 0.f;
-    // slab 0 into buffer 0, slab 1 into the registers
-#pragma unroll
-    for (int u = 0; u < NU; ++u) gload(0, u);
-#pragma unroll
-    for (int u = 0; u < NU; ++u) lstore(0, u);
-#pragma unroll
-    for (int u = 0; u < NU; ++u) gload(1, u);
-    __syncthreads();
-
-    // slab kt from buffer kt % 2; STORE: the registers (slab kt + 1) go to the
-    // other buffer; LOAD: slab kt + 2 refills them. Compile-time flags keep the
-    // k loop one branch-free block.
-    auto slab = [&](int64_t kt, auto store_next, auto load_after) {
-        constexpr bool STORE = decltype(store_next)::value, LOAD = decltype(load_after)::value;
-        const int cur = (int) (kt & 1);
-        const float* ac = As[cur];
-        const float* bc = Bs[cur];
-        if constexpr (PL::PRIO) __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int t4 = 0; t4 < BK / 4; ++t4) {
-            const int k0 = 4 * t4 + 2 * half;
-            float2 av[DB_TI], bv[DB_TJ];
-#pragma unroll
-            for (int x = 0; x < DB_TI; ++x) av[x] = PA::pair(ac, k0, (wi * DB_TI + x) * 32 + col);
-#pragma unroll
-            for (int y = 0; y < DB_TJ; ++y) bv[y] = PB::pair(bc, k0, (wj * DB_TJ + y) * 32 + col);
-#pragma unroll
-            for (int x = 0; x < DB_TI; ++x)
-#pragma unroll
-                for (int y = 0; y < DB_TJ; ++y) {
-                    acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[y].x, av[x].x, acc[x][y], 0, 0, 0);
-                    acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[y].y, av[x].y, acc[x][y], 0, 0, 0);
-                }
-            if constexpr (STORE) {
-                if (t4 >= PL::S0 && t4 < PL::S0 + NU) lstore(cur ^ 1, t4 - PL::S0);
-            }
-            if constexpr (LOAD) {
-                if (t4 >= PL::L0 && t4 < PL::L0 + NU) gload(kt + 2, t4 - PL::L0);
-            }
-        }
-        if constexpr (PL::PRIO) __builtin_amdgcn_s_setprio(0);
-        __syncthreads();
-    };
-    using yes = std::integral_constant<bool, true>;
-    using no = std::integral_constant<bool, false>;
-    // (nk >= 2 here; the guards also give the compiler the block layout that
-    // measured 146 us for dX against 149 us without them, the loop unchanged)
-    for (int64_t kt = 0; kt + 2 < nk; ++kt) slab(kt, yes{}, yes{});
-    if (nk >= 2) slab(nk - 2, yes{}, no{});
-    if (nk >= 1) slab(nk - 1, no{}, no{});
-
-    // accumulator register v of tile (x, y) holds dst row i = i0 + (wi TI + x) 32
-    // + col and column j = j0 + (wj TJ + y) 32 + 8 (v / 4) + 4 half + v % 4
-    auto out = [&](int x, int y, int v) -> float* {
-        const int64_t i = i0 + (wi * DB_TI + x) * 32 + col;
-        const int64_t j = j0 + (wj * DB_TJ + y) * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
-        return i < p.M && j < p.N ? (float*) (d + i * p.d_nb0 + j * p.d_nb1) : nullptr;
-    };
-    if constexpr (SPLIT > 1) {
-        // the parts meet in dst (ticket_first and the protocol it begins, common.h)
-        uint32_t* tk = p.tickets + 2 * (tile * (DB_WI * DB_WJ) + wave);
-        if (ticket_first(tk, lane)) {
-#pragma unroll
-            for (int x = 0; x < DB_TI; ++x)
-#pragma unroll
-                for (int y = 0; y < DB_TJ; ++y)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v)
-                        if (float* o = out(x, y, v))
-                            __hip_atomic_store(o, acc[x][y][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            ticket_publish(tk, lane);
-            return;
-        }
-        ticket_wait(tk, lane);
-#pragma unroll
-        for (int x = 0; x < DB_TI; ++x)
-#pragma unroll
-            for (int y = 0; y < DB_TJ; ++y)
-#pragma unroll
-                for (int v = 0; v < 16; ++v)
-                    if (float* o = out(x, y, v))
-                        __hip_atomic_fetch_add(o, acc[x][y][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ticket_clear(tk, lane);
-    } else if constexpr (ACC) {
-        // d + v, one 32 x 32 block at a time with its 16 old values read before
-        // any store, through a buffer resource over the dst plane (as k_mul_mat's
-        // ACC epilogue; the tile is whole, so one lane offset and uniform
-        // multiples of nb1 address all 16)
-        const __amdgpu_buffer_rsrc_t rd =
-            __builtin_amdgcn_make_buffer_rsrc((void*) d, (short) 0, (int) p.d_span, MM_RSRC_WORD3);
-#pragma unroll
-        for (int x = 0; x < DB_TI; ++x) {
-            const int64_t i = i0 + (wi * DB_TI + x) * 32 + col;
-#pragma unroll
-            for (int y = 0; y < DB_TJ; ++y) {
-                const int64_t jb = j0 + (wj * DB_TJ + y) * 32 + 4 * half;
-                const uint32_t vo = (uint32_t) (i * p.d_nb0 + jb * p.d_nb1);
-                float old[16];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const uint32_t so = (uint32_t) ((8 * (v >> 2) + (v & 3)) * p.d_nb1);
-                    old[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, vo, so, 0));
-                }
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const uint32_t so = (uint32_t) ((8 * (v >> 2) + (v & 3)) * p.d_nb1);
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, old[v] + acc[x][y][v]), rd, vo,
-                                                          so, 0);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-    } else {
-        // non-temporal: dst is not read again by this launch. The tile is
-        // whole, so no element needs a bounds check; with out()'s check (and
-        // its branches) dW took 145-148 us instead of 131
-#pragma unroll
-        for (int x = 0; x < DB_TI; ++x)
-#pragma unroll
-            for (int y = 0; y < DB_TJ; ++y)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int64_t i = i0 + (wi * DB_TI + x) * 32 + col;
-                    const int64_t j = j0 + (wj * DB_TJ + y) * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
-                    __builtin_nontemporal_store(acc[x][y][v], (float*) (d + i * p.d_nb0 + j * p.d_nb1));
-                }
-    }
-}
-
-// Launches k_mul_mat_db when the shape fits it (whole tiles and slabs, float4
-// loaders, the K parts' ticket words in p.tickets when SPLIT is 2); returns
-// -1 (launching nothing) otherwise.
-template <int SPLIT, bool ACC>
-int launch_db(MMArgs& p, int am, int bm, int64_t planes, hipStream_t stream) {
-    static_assert(DbPlan<SPLIT, K_CONTIG>::BK == DbPlan<SPLIT, R_CONTIG>::BK, "one slab depth per K split");
-    constexpr int BK = DbPlan<SPLIT, K_CONTIG>::BK;
-    if (p.M % DB_BM != 0 || p.N % DB_BN != 0 || p.K % (2 * BK * SPLIT) != 0 || am == GENERIC || bm == GENERIC)
-        return -1;
-    p.tiles_i = p.M / DB_BM;
-    p.tiles_j = p.N / DB_BN;
-    p.xcd_planes = planes % 8 == 0 ? 1 : 0;
-    p.d_span = (p.M - 1) * p.d_nb0 + (p.N - 1) * p.d_nb1 + 4;
-    const int64_t grid = p.tiles_i * p.tiles_j * planes * SPLIT;
-    if (grid > 0x7FFFFFFF) return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) grid);
-#define TRC_MM_DB(A, B) \
-    if (am == A && bm == B) \
-        hipLaunchKernelGGL((k_mul_mat_db<A, B, SPLIT, ACC>), dim3((unsigned) grid), dim3(DB_THREADS), 0, stream, p);
-    TRC_MM_DB(K_CONTIG, K_CONTIG)
-    TRC_MM_DB(K_CONTIG, R_CONTIG)
-    TRC_MM_DB(R_CONTIG, K_CONTIG)
-    TRC_MM_DB(R_CONTIG, R_CONTIG)
-#undef TRC_MM_DB
-    return check_launch("mul_mat_f32 (double-buffered slabs)");
 }
 
 // ---------------------------------------------------------------- few columns
@@ -962,24 +547,24 @@ int pick_mode(const trc_hip_tensor& t, int64_t rows) {
     return GENERIC;
 }
 
-template <int WI, int WJ, int TI, int TJ, int BK, int AM, int BMO, int SPLIT, bool ACC, bool KI = false>
+template <int WI, int WJ, int TI, int TJ, int BK, int AM, int BMO, bool ACC>
 int launch_cfg(MMArgs& p, int64_t planes, hipStream_t stream) {
     constexpr int BM = WI * TI * 32, BN = WJ * TJ * 32;
     p.tiles_i = (p.M + BM - 1) / BM;
     p.tiles_j = (p.N + BN - 1) / BN;
-    const int64_t grid = p.tiles_i * p.tiles_j * planes * SPLIT;
+    const int64_t grid = p.tiles_i * p.tiles_j * planes;
     if (grid > 0x7FFFFFFF) return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) grid);
     p.xcd_planes = planes % 8 == 0 ? 1 : 0;
     p.d_span = (p.M - 1) * p.d_nb0 + (p.N - 1) * p.d_nb1 + 4;
-    hipLaunchKernelGGL((k_mul_mat<WI, WJ, TI, TJ, BK, AM, BMO, SPLIT, ACC, KI>), dim3((unsigned) grid),
+    hipLaunchKernelGGL((k_mul_mat<WI, WJ, TI, TJ, BK, AM, BMO, ACC>), dim3((unsigned) grid),
                        dim3(WI * WJ * 64), 0, stream, p);
     return check_launch("mul_mat_f32");
 }
 
-template <int WI, int WJ, int TI, int TJ, int BK, int SPLIT, bool ACC = false>
+template <int WI, int WJ, int TI, int TJ, int BK, bool ACC>
 int dispatch_modes(MMArgs& p, int am, int bm, int64_t planes, hipStream_t s) {
 #define TRC_MM_CASE(A, B) \
-    if (am == A && bm == B) return launch_cfg<WI, WJ, TI, TJ, BK, A, B, SPLIT, ACC>(p, planes, s);
+    if (am == A && bm == B) return launch_cfg<WI, WJ, TI, TJ, BK, A, B, ACC>(p, planes, s);
     TRC_MM_CASE(K_CONTIG, K_CONTIG)
     TRC_MM_CASE(K_CONTIG, R_CONTIG)
     TRC_MM_CASE(K_CONTIG, GENERIC)
@@ -999,6 +584,9 @@ int launch_mul_mat_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const t
                        hipStream_t stream, bool accumulate) {
     MMArgs p;
     p.tickets = nullptr;
+    p.slots = nullptr;
+    p.parts = 1;
+    p.part = 0;
     p.a = (const uint8_t*) a.data;
     p.b = (const uint8_t*) b.data;
     p.d = (uint8_t*) d.data;
@@ -1038,44 +626,27 @@ int launch_mul_mat_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const t
         return launch_skinny_nt<4, 1>(s, sbm, planes, stream);
     }
 
-    // Large tiles when they still give every CU at least two workgroups. With
-    // between half and two tiles per CU and a long K, large tiles with K in two
-    // parts (into a contiguous dst; the parts meet through ticket words in the
-    // stream's workspace); otherwise 64x64 tiles.
+    // Tiles of 64 x 64 with the FP32 instructions take 5 us and 0.7 us per 32 k
+    // (0.85 to 1.1 us where an operand loads element by element), up to about 400 of
+    // them; the bf16 tiles are taken where their model's time is less (measured,
+    // FP32 -> bf16: 768 x 2048 x 256 21.1 -> 19.1, 512 x 512 x 515 unaligned 24.6
+    // -> 16.1; 512 x 512 x 512 15.1 -> 15.7, 300 x 300 x 300 11.0 -> 14.0).
+    const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * planes;
+    if (mm_bf3_fits(p)) {
+        // added into dst: K stays in one part
+        B3Plan plan = mm_bf3_plan(p, planes, accumulate ? 1 : 8);
+        const double slabs = (double) ((p.K + 31) / 32);
+        const double us64 = 5 + (am == GENERIC || bm == GENERIC ? 0.85 : 0.7) * slabs * (tiles64 > 400 ? (double) tiles64 / 400 : 1.0);
+        if (plan.us < us64) return launch_mm_bf3(p, planes, plan.groups, plan.parts, accumulate, stream);
+    }
+    // Large tiles when they still give every CU at least two workgroups.
     const int64_t big_tiles = ((p.M + 127) / 128) * ((p.N + 127) / 128) * planes;
-    if (accumulate) {
-        // K stays in one part: the large tiles when they fill the CUs twice
-        // (double-buffered when whole), else 64 x 64
-        if (big_tiles >= 512) {
-            const int drc = launch_db<1, true>(p, am, bm, planes, stream);
-            if (drc >= 0) return drc;
-            return dispatch_modes<2, 2, 2, 2, 16, 1, true>(p, am, bm, planes, stream);
-        }
-        return dispatch_modes<2, 2, 1, 1, 32, 1, true>(p, am, bm, planes, stream);
-    }
     if (big_tiles >= 512) {
-        const int drc = launch_db<1, false>(p, am, bm, planes, stream);
-        if (drc >= 0) return drc;
-        return dispatch_modes<2, 2, 2, 2, 16, 1>(p, am, bm, planes, stream);
+        return accumulate ? dispatch_modes<2, 2, 2, 2, 16, true>(p, am, bm, planes, stream)
+                          : dispatch_modes<2, 2, 2, 2, 16, false>(p, am, bm, planes, stream);
     }
-    const bool dense_dst = p.d_nb0 == 4 && p.d_nb1 == 4 * p.M && p.d_nb2 == p.d_nb1 * p.N &&
-                           p.d_nb3 == p.d_nb2 * b.ne[2];
-    if (dense_dst && p.K >= 1024 && 2 * big_tiles >= device_cus()) {
-        static_assert(511 * 8 * 2 <= MM_TICKETS, "two ticket words per wave of under 512 tiles");
-        const int rc = mm_stream_tickets(stream, &p.tickets);
-        if (rc != TRC_HIP_OK) return rc;
-        // whole tiles and slabs with float4 loaders: double-buffered slabs
-        const int drc = launch_db<2, false>(p, am, bm, planes, stream);
-        if (drc >= 0) return drc;
-        // a transposed src0 against a k-contiguous src1 (the dX product of a
-        // Linear layer): k-paired LDS planes for src1, 4 % faster there; 1.5 %
-        // slower with both operands k-contiguous (the forward product)
-        if (am == R_CONTIG && bm == K_CONTIG) {
-            return launch_cfg<2, 4, 2, 1, 32, R_CONTIG, K_CONTIG, 2, false, true>(p, planes, stream);
-        }
-        return dispatch_modes<2, 4, 2, 1, 32, 2>(p, am, bm, planes, stream);
-    }
-    return dispatch_modes<2, 2, 1, 1, 32, 1>(p, am, bm, planes, stream);
+    return accumulate ? dispatch_modes<2, 2, 1, 1, 32, true>(p, am, bm, planes, stream)
+                      : dispatch_modes<2, 2, 1, 1, 32, false>(p, am, bm, planes, stream);
 }
 
 }  // namespace trc_hip

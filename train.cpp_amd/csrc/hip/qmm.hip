@@ -1025,6 +1025,7 @@ struct StreamWs {
     std::thread::id thread;  // only for hipStreamPerThread
     uint8_t* ptr;
     uint64_t last_use;
+    uint8_t* slots;  // the K-split mul_mat's slots, allocated by the first call that needs them
 };
 std::vector<StreamWs>& stream_workspaces() {
     static std::vector<StreamWs> v;
@@ -1112,16 +1113,68 @@ int qm_stream_workspace(hipStream_t s, uint8_t** ws) {
         (void) hipFree(p);
         return frc;
     }
-    v.push_back({dev, s, tid, (uint8_t*) p, ++g_ws_clock});
+    v.push_back({dev, s, tid, (uint8_t*) p, ++g_ws_clock, nullptr});
     *ws = (uint8_t*) p;
     return TRC_HIP_OK;
 }
 
-int mm_stream_tickets(hipStream_t s, uint32_t** tickets) {
-    uint8_t* ws = nullptr;
-    const int rc = qm_stream_workspace(s, &ws);
+int mm_stream_scratch(hipStream_t s, size_t slots, uint32_t** tickets, float** sums) {
+    *tickets = nullptr;
+    *sums = nullptr;
+    if (slots > MM_SLOTS) return fail(TRC_HIP_E_INVALID, "mul_mat: %zu slots", slots);
+    int dev = 0;
+    int rc = current_device(&dev);
     if (rc != TRC_HIP_OK) return rc;
-    *tickets = (uint32_t*) (ws + QM_WS_BYTES);
+    const std::thread::id tid = stream_thread(s);
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    std::vector<StreamWs>& v = stream_workspaces();
+    int on_dev = 0;
+    StreamWs* own = nullptr;
+    for (StreamWs& w : v) {
+        if (w.dev != dev) continue;
+        ++on_dev;
+        if (w.stream == s && w.thread == tid) own = &w;
+    }
+    if (own == nullptr || (slots > 0 && own->slots == nullptr)) {
+        // Something has to be allocated: not for a stream under capture (or one
+        // that a capture elsewhere bars), nor by taking another stream's.
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+            (void) hipGetLastError();
+            return TRC_HIP_OK;
+        }
+        if (own == nullptr && on_dev >= QM_STREAM_WS) return TRC_HIP_OK;
+        // a capture on another thread is left alone by the allocation
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+        hipError_t e = hipSuccess;
+        if (own == nullptr) {
+            void* p = nullptr;
+            e = hipMalloc(&p, QM_WS_BYTES + MM_TICKETS * sizeof(uint32_t));
+            if (e == hipSuccess) {
+                rc = launch_fill_f32((float*) ((uint8_t*) p + QM_WS_BYTES), 0.f, MM_TICKETS, s);
+                if (rc == TRC_HIP_OK) {
+                    v.push_back({dev, s, tid, (uint8_t*) p, 0, nullptr});
+                    own = &v.back();
+                } else {
+                    (void) hipFree(p);
+                }
+            }
+        }
+        if (own != nullptr && slots > 0) {
+            void* p = nullptr;
+            e = hipMalloc(&p, MM_SLOTS * 65536);
+            if (e == hipSuccess) own->slots = (uint8_t*) p;
+        }
+        if (swapped) (void) hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess || rc != TRC_HIP_OK) {  // no memory: the parts run one after another
+            (void) hipGetLastError();
+            return TRC_HIP_OK;
+        }
+    }
+    own->last_use = ++g_ws_clock;
+    *tickets = (uint32_t*) (own->ptr + QM_WS_BYTES);
+    *sums = (float*) own->slots;
     return TRC_HIP_OK;
 }
 
@@ -1138,6 +1191,10 @@ int qm_release_stream(hipStream_t s) {
         rc = hip_error(hipStreamSynchronize(s), "qmatvec_release_stream: hipStreamSynchronize");
         if (rc != TRC_HIP_OK) return rc;
         rc = hip_error(hipFree(v[i].ptr), "qmatvec_release_stream: hipFree");
+        if (v[i].slots != nullptr) {
+            const int src = hip_error(hipFree(v[i].slots), "qmatvec_release_stream: hipFree");
+            if (rc == TRC_HIP_OK) rc = src;
+        }
         v.erase(v.begin() + (long) i);
         return rc;
     }
