@@ -89,3 +89,26 @@ def test_forced_error_hook(hip):
         assert "forced" in H.last_error()
     finally:
         del os.environ["TRC_HIP_FORCE_ERROR"]
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 5, 128), (1, 4, 7, 4), (3, 2, 9, 33), (1, 1, 1, 1), (2, 12, 333, 64), (1, 1, 3000, 3)])
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16, np.float32, np.int64])
+def test_cpy_permuted_planes(hip, shape, dtype):
+    """Rows that run along ne0 on both sides with their planes permuted (merged heads),
+    in whole 16-byte pieces and not, and into a wider dst, for every element size."""
+    announce(f"abi cpy permuted {shape} {np.dtype(dtype).name}")
+    code = {1: 24, 2: 1, 4: 0, 8: 27}[np.dtype(dtype).itemsize]
+    rng = np.random.default_rng(31)
+    a = rng.integers(0, 200, shape).astype(dtype)
+    src = Dev(a)
+    view = np.swapaxes(src.base, 1, 2)
+    for pad in (0, 1):
+        wide = np.zeros(view.shape[:-1] + (view.shape[-1] + pad,), dtype)
+        out = Dev(wide)
+        H.cpy(src.tensor(view, code), out.tensor(out.base[..., :view.shape[-1]], code))
+        H.sync()
+        got = out.read()
+        assert np.array_equal(got[..., :view.shape[-1]], view)
+        assert not got[..., view.shape[-1]:].any()
+        out.free()
+    src.free()

@@ -97,6 +97,20 @@ __device__ __forceinline__ void ticket_wait_all(uint32_t* tk, int lane, uint32_t
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// Division of a number under 2^31 by a fixed one as a multiply and a shift (Granlund
+// and Montgomery, "Division by invariant integers using multiplication", 1994).
+struct FastDiv {
+    uint32_t d, m, s;
+};
+inline FastDiv fast_div(int64_t d) {
+    uint32_t s = 0;
+    while (((uint64_t) 1 << s) < (uint64_t) d) ++s;
+    return {(uint32_t) d, (uint32_t) ((((uint64_t) 1 << 32) * (((uint64_t) 1 << s) - (uint64_t) d)) / (uint64_t) d + 1), s};
+}
+__device__ __forceinline__ uint32_t div_by(uint32_t n, FastDiv f) {
+    return (uint32_t) (((uint64_t) __umulhi(n, f.m) + n) >> f.s);
+}
+
 // Launch-side error reporting, implemented in abi.hip.
 int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);
