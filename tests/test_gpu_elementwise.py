@@ -374,3 +374,102 @@ def test_sqr_and_scale_reject_bad_shapes(hip):
         H.scale_f32(da.tensor(), out.tensor(), 2.0)
     da.free()
     out.free()
+
+
+@pytest.mark.parametrize("shape,cut", [((130, 777), None), ((1, 64), None), ((9, 63), None), ((17, 65), None),
+                                       ((8, 256), None), ((7, 255), None), ((3, 5, 9, 272), None), ((40, 1030), 1027),
+                                       ((9000, 66), None), ((8256, 64), None)])
+def test_sum_staged_rows_bitwise(hip, shape, cut):
+    """Rows streamed through LDS, aligned and not: lengths at the edges of its chunks
+    of 256 and groups of 16, counts at the edges of its 8 rows a workgroup and of the
+    batches the last workgroup adds; twice, so that the ticket is left clear."""
+    announce(f"sum staged rows {shape} cut {cut}")
+    rng = np.random.default_rng(28)
+    a = (rng.standard_normal(shape) * 10.0 ** rng.integers(-3, 4, shape)).astype(np.float32)
+    av = a if cut is None else a[..., :cut]
+    want = bits(O.sum_all(av))
+    assert bits(gpu_sum(a, av)) == want
+    assert bits(gpu_sum(a, av)) == want
+    t = np.ascontiguousarray(np.swapaxes(a, -1, -2))  # strided rows
+    assert bits(gpu_sum(t, np.swapaxes(t, -1, -2)[..., :av.shape[-1]])) == want
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1024, 1027, 100_001])
+@pytest.mark.parametrize("off", [0, 1])
+def test_contiguous_elementwise_bitwise(hip, n, off):
+    """Contiguous operands as one run of floats: lengths at the edges of a float4 and
+    of a workgroup, and operands one float off 16-byte alignment."""
+    announce(f"contiguous element-wise n={n} off={off}")
+    rng = np.random.default_rng(n)
+    a, b = (rng.standard_normal(n + off).astype(np.float32) for _ in range(2))
+    da, db, dd = Dev(a), Dev(b), empty((n + 4,))
+    at, bt = da.tensor(da.base[off:]), db.tensor(db.base[off:])
+    dt = H.tensor(dd.ptr + 4 * off, [n, 1, 1, 1], H.contiguous_nb([n, 1, 1, 1]))
+    x, y = a[off:], b[off:]
+    for call, want in ((lambda: H.add_f32(at, bt, dt), x + y), (lambda: H.mul_f32(at, bt, dt), x * y),
+                       (lambda: H.sqr_f32(at, dt), x * x), (lambda: H.scale_f32(at, dt, 0.3), x * np.float32(0.3))):
+        H.fill_f32(dd.ptr, 7.0, n + 4)
+        call()
+        H.sync()
+        got = dd.read()
+        assert np.array_equal(got[off:off + n].view(np.uint32), want.view(np.uint32))
+        assert np.all(got[:off] == 7.0) and np.all(got[off + n:] == 7.0)
+    for d in (da, db, dd):
+        d.free()
+
+
+@pytest.mark.parametrize("ashape,dshape", [((2, 12, 33, 64), (2, 4, 33, 64)), ((4, 2, 6, 5), (2, 1, 3, 5)),
+                                           ((1, 64, 3, 7), (1, 1, 3, 7)), ((1, 65, 3, 8), (1, 1, 3, 8)),
+                                           ((3, 3, 7, 12), (1, 1, 1, 12)), ((2, 2, 40, 8), (2, 2, 1, 8))])
+@pytest.mark.parametrize("swap", [False, True])
+def test_repeat_back_few_terms_bitwise(hip, ashape, dshape, swap):
+    """Outputs of few terms, over every dimension but ne0, from contiguous and from
+    permuted operands; 65 terms take the kernel for many."""
+    announce(f"repeat_back few {ashape} {dshape} swap={swap}")
+    rng = np.random.default_rng(29)
+    a = (rng.standard_normal(ashape) * 10.0 ** rng.integers(-2, 3, ashape)).astype(np.float32)
+    base = np.ascontiguousarray(np.swapaxes(a, 1, 2)) if swap else a
+    da, dd = Dev(base), empty(dshape)
+    H.repeat_back_f32(da.tensor(np.swapaxes(da.base, 1, 2) if swap else da.base), dd.tensor())
+    H.sync()
+    got = dd.read()
+    want = np.zeros(dshape, np.float32)
+    r = [x // y for x, y in zip(ashape, dshape)]
+    for k3 in range(r[0]):
+        for k2 in range(r[1]):
+            for k1 in range(r[2]):
+                want = want + a[k3 * dshape[0]:(k3 + 1) * dshape[0], k2 * dshape[1]:(k2 + 1) * dshape[1],
+                                k1 * dshape[2]:(k1 + 1) * dshape[2]]
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    da.free()
+    dd.free()
+
+
+@pytest.mark.parametrize("bshape,pads", [((3, 4, 5, 7), (0, 0, 0)), ((2, 3, 6, 8), (0, 0, 0)), ((2, 3, 6, 8), (4, 0, 0)),
+                                         ((2, 3, 6, 8), (1, 0, 0)), ((2, 3, 6, 7), (0, 3, 0)), ((1, 1, 9, 16), (0, 8, 32))])
+@pytest.mark.parametrize("offset", [0, 4, 16])
+def test_acc_regions_bitwise(hip, bshape, pads, offset):
+    """Regions as dense as b, with padded rows and planes, at offsets on and off 16
+    bytes: one run of floats, float4 rows and single floats."""
+    announce(f"acc region {bshape} pads {pads} offset {offset}")
+    rng = np.random.default_rng(33)
+    b = rng.standard_normal(bshape).astype(np.float32)
+    n0, n1, n2, n3 = bshape[::-1]
+    nb1 = 4 * (n0 + pads[0])
+    nb2 = nb1 * n1 + 4 * pads[1]
+    nb3 = nb2 * n2 + 4 * pads[2]
+    total = (offset + nb3 * n3 + 64) // 4
+    a = rng.standard_normal(total).astype(np.float32)
+    want = a.copy()
+    for i3 in range(n3):
+        for i2 in range(n2):
+            for i1 in range(n1):
+                at = (offset + i1 * nb1 + i2 * nb2 + i3 * nb3) // 4
+                want[at:at + n0] = want[at:at + n0] + b[i3, i2, i1]
+    da, db = Dev(a), Dev(b)
+    t = da.tensor()
+    H.acc_f32(t, db.tensor(), t, nb1, nb2, nb3, offset, True)
+    H.sync()
+    assert np.array_equal(da.read().view(np.uint32), want.view(np.uint32))
+    da.free()
+    db.free()

@@ -125,6 +125,34 @@ __global__ __launch_bounds__(EW_THREADS) void k_unary4(const uint8_t* __restrict
     }
 }
 
+// The same operations where every operand is one contiguous run of n floats (16-byte
+// aligned): float4s with no rows to find, which rows of odd lengths leave to single
+// floats otherwise, and every lane busy whatever ne0 is. NT: the result is larger
+// than the caches and is stored past them (268 MB scaled: 102 -> 85 us).
+enum class FlatOp { ADD, MUL, SQR, SCALE };
+constexpr int64_t FLAT_NT = (int64_t) 32 << 20;  // floats
+template <FlatOp OP, bool NT>
+__global__ __launch_bounds__(EW_THREADS) void k_flat(const f4* a, const f4* b, f4* d, int64_t n, float s) {
+    auto one = [&](auto x, auto y) {
+        if constexpr (OP == FlatOp::ADD) return x + y;
+        else if constexpr (OP == FlatOp::MUL) return x * y;
+        else if constexpr (OP == FlatOp::SQR) return x * x;
+        else return x * s;
+    };
+    constexpr bool TWO = OP == FlatOp::ADD || OP == FlatOp::MUL;
+    const int64_t q = (int64_t) blockIdx.x * EW_THREADS + threadIdx.x;
+    if (q < n / 4) {
+        const f4 va = a[q], v = one(va, TWO ? b[q] : va);
+        if constexpr (NT) __builtin_nontemporal_store(v, d + q);
+        else d[q] = v;
+    } else if (q == n / 4) {  // the last n % 4
+        for (int64_t i = n / 4 * 4; i < n; ++i) {
+            const float x = ((const float*) a)[i];
+            ((float*) d)[i] = one(x, TWO ? ((const float*) b)[i] : x);
+        }
+    }
+}
+
 // k_repeat for a dst whose rows are 16-byte aligned with nb0 == 4 and ne0 % 4 ==
 // 0: one row of dst per workgroup pass, four floats per lane and store.
 __global__ __launch_bounds__(EW_THREADS) void k_repeat4(const uint8_t* __restrict__ a, Shape4 sa,
@@ -171,12 +199,12 @@ __global__ __launch_bounds__(EW_THREADS) void k_repeat(const uint8_t* __restrict
 // double in element order, the row sums added in double in row order (i1
 // fastest, then i2, i3), one rounding to float at the end.
 //
-// Two launches. k_sum_rows: one lane per row, its row's sequential double sum
-// (the chain cannot be split without changing the rounding), with the row's
-// next SR_AHEAD loads issued ahead of the adds, from addresses clamped into the
-// row so no branch waits on them; the row sums go to a workspace. k_sum_combine:
-// one wave adds them in row order. k_sum (one workgroup, no workspace) serves
-// the row counts the workspace cannot hold.
+// Rows of 64 elements and more (k_sum_rows_lds) stream through LDS and meet in the
+// workgroup that finishes last. Shorter rows take two launches: k_sum_rows, one
+// lane per row with the row's next SR_AHEAD loads issued ahead of the adds (from
+// addresses clamped into the row, so no branch waits on them), then k_sum_combine,
+// one wave that adds the row sums in row order. k_sum (one workgroup, no
+// workspace) serves the row counts the workspace cannot hold.
 constexpr int SR_THREADS = 64;
 constexpr int SR_AHEAD = 32;
 
@@ -229,67 +257,111 @@ __global__ __launch_bounds__(SR_THREADS) void k_sum_rows(const uint8_t* __restri
     part[r] = s;
 }
 
-// k_sum_rows for 16-byte aligned rows (nb0 == 4), with the loads spread over a
-// whole workgroup: SB_ROWS rows per workgroup stream through an LDS ring of
-// SB_D chunks of SB_C floats per row, loaded by all SB_THREADS threads (1 KB
-// runs per row) SB_D - 1 chunks ahead of the lanes that hold the rows' sums;
-// lane r of wave 0 adds row r's chunk in element order. With SB_D >= 3 one
-// barrier per chunk separates a slot's reads from its next fill. The threads
-// that stage a chunk convert it to double (exact) as they store it, so the
-// lanes on the chain issue only the adds (configuration 3's loss: 29.1 ->
-// 27.0 us per launch). What remains is the chain itself: each dependent
-// v_add_f64 waits ~15 cycles for the one before, 4096 of them per row.
+// Row sums with the loads spread over a whole workgroup: SB_ROWS rows per
+// workgroup stream through an LDS ring of SB_D chunks of SB_C elements per row,
+// loaded by all SB_THREADS threads (float4s where VEC: nb0 == 4, whole float4s, rows
+// 16-byte aligned; else element by element, still in runs along the row) SB_D - 1
+// chunks ahead of the lanes that hold the rows' sums; lane r of wave 0 adds row r's
+// chunk in element order. With SB_D >= 3 one barrier per chunk separates a slot's
+// reads from its next fill. The threads that stage a chunk convert it to double
+// (exact) as they store it, so the lanes on the chain issue only the adds, and
+// store zeros past the row's end, which change no sum (it is never -0: it starts
+// from +0). What remains is the chain itself: each dependent v_add_f64 waits ~15
+// cycles for the one before. 130 rows of 777 unaligned floats: 50 us with one lane
+// per row, 13 here.
+// The workgroup that takes the last ticket adds the row sums in row order (512
+// rows of 4096 40.0 us with a launch of its own for that, 37.2 here).
 constexpr int SB_ROWS = 8;
 constexpr int SB_THREADS = 256;
 constexpr int SB_C = 256;
 constexpr int SB_LD = SB_C + 2;  // padded row (in doubles) of an LDS slot: rows 4 banks apart
+constexpr int SB_MIN = 64;       // shorter rows: one lane each
 typedef double sb_d2 __attribute__((ext_vector_type(2)));
 constexpr int SB_D = 4;
-constexpr int SB_PER = SB_ROWS * SB_C / 4 / SB_THREADS;  // float4 loads per thread and chunk
-static_assert(SB_PER * SB_THREADS * 4 == SB_ROWS * SB_C, "a chunk is whole float4s per thread");
+constexpr int SB_RING = SB_D * SB_ROWS * SB_LD;
 
-__global__ __launch_bounds__(SB_THREADS) void k_sum_rows_lds(const uint8_t* __restrict__ a, Shape4 sa,
-                                                             double* __restrict__ part) {
-    __shared__ __attribute__((aligned(16))) double ring[SB_D * SB_ROWS * SB_LD];
+// s + the first n doubles (n a multiple of 16) at p, in order: the next 16 are read
+// from LDS while the current 16 are added
+__device__ __forceinline__ double sum_chain(double s, const double* p, int n) {
+    const sb_d2* q = (const sb_d2*) p;
+    sb_d2 cur[8], nxt[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) cur[k] = q[k];
+    for (int g = 16; g < n; g += 16) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) nxt[k] = q[g / 2 + k];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            s = s + cur[k].x;
+            s = s + cur[k].y;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) cur[k] = nxt[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        s = s + cur[k].x;
+        s = s + cur[k].y;
+    }
+    return s;
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(SB_THREADS) void k_sum_rows_lds(const uint8_t* __restrict__ a, Shape4 sa, double* part,
+                                                             uint32_t* ticket, float* __restrict__ d) {
+    constexpr int W = VEC ? 4 : 1;                         // elements per load
+    constexpr int PER = SB_ROWS * SB_C / W / SB_THREADS;   // loads per thread and chunk
+    static_assert(PER * SB_THREADS * W == SB_ROWS * SB_C, "a chunk is whole loads per thread");
+    static_assert(SB_C / W <= SB_THREADS, "a thread's loads are whole rows apart");
+    __shared__ __attribute__((aligned(16))) double ring[SB_RING];
+    __shared__ uint32_t order;
     const int64_t rows = sa.ne[1] * sa.ne[2] * sa.ne[3];
     const int64_t r0 = (int64_t) blockIdx.x * SB_ROWS;
     const int64_t n = sa.ne[0];
-    const int64_t n4 = n / 4;
     const int64_t chunks = (n + SB_C - 1) / SB_C;
     const int tid = threadIdx.x;
-    // this thread's float4s of a chunk: row e / (SB_C / 4), float4 e % (SB_C / 4)
-    const f4* src[SB_PER];
-    int lrow[SB_PER], lq[SB_PER];
+    // load u of this thread: row tid / (SB_C / W) + u * (rows a pass covers), the same place in every row
+    const int lq = tid % (SB_C / W), lr = tid / (SB_C / W);
+    constexpr int STEP = SB_THREADS / (SB_C / W);
+    const uint8_t* src[PER];
 #pragma unroll
-    for (int u = 0; u < SB_PER; ++u) {
-        const int e = tid + SB_THREADS * u;
-        lrow[u] = e / (SB_C / 4);
-        lq[u] = e % (SB_C / 4);
-        int64_t r = r0 + lrow[u];
+    for (int u = 0; u < PER; ++u) {
+        int64_t r = r0 + lr + u * STEP;
         r = r < rows ? r : rows - 1;  // rows past the end re-read the last; nobody adds them
         const int64_t i1 = r % sa.ne[1], i2 = (r / sa.ne[1]) % sa.ne[2], i3 = r / (sa.ne[1] * sa.ne[2]);
-        src[u] = (const f4*) (a + i1 * sa.nb[1] + i2 * sa.nb[2] + i3 * sa.nb[3]);
+        src[u] = a + i1 * sa.nb[1] + i2 * sa.nb[2] + i3 * sa.nb[3];
     }
-    // float4 q of a row covers elements 4q .. 4q + 3 (n % 4 == 0 on this path); a
-    // float4 past the row's end is read from the row's last (valid) and never added
-    auto load = [&](int64_t c, f4 (&v)[SB_PER]) {
+    // elements past the row's end are read from its last ones and staged as zeros
+    auto load = [&](int64_t c, float (&v)[PER][W]) {
+        const int64_t e = c * SB_C + lq * W;
+        const int64_t at = (e < n ? e : n - W) * (VEC ? 4 : sa.nb[0]);
 #pragma unroll
-        for (int u = 0; u < SB_PER; ++u) {
-            const int64_t q = c * (SB_C / 4) + lq[u];
-            v[u] = src[u][q < n4 ? q : n4 - 1];
+        for (int u = 0; u < PER; ++u) {
+            if constexpr (VEC) {
+                const f4 q = *(const f4*) (src[u] + at);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[u][k] = q[k];
+            } else {
+                v[u][0] = *(const float*) (src[u] + at);
+            }
         }
     };
-    auto store = [&](int64_t c, const f4 (&v)[SB_PER]) {
+    auto store = [&](int64_t c, const float (&v)[PER][W]) {
         double* slot = ring + (int) (c % SB_D) * SB_ROWS * SB_LD;
+        const bool in = c * SB_C + lq * W < n;
 #pragma unroll
-        for (int u = 0; u < SB_PER; ++u) {
-            double* dst = slot + lrow[u] * SB_LD + 4 * lq[u];
-            *(sb_d2*) dst = sb_d2{(double) v[u].x, (double) v[u].y};
-            *(sb_d2*) (dst + 2) = sb_d2{(double) v[u].z, (double) v[u].w};
+        for (int u = 0; u < PER; ++u) {
+            double* o = slot + (lr + u * STEP) * SB_LD + W * lq;
+            if constexpr (VEC) {
+                *(sb_d2*) o = sb_d2{in ? (double) v[u][0] : 0.0, in ? (double) v[u][1] : 0.0};
+                *(sb_d2*) (o + 2) = sb_d2{in ? (double) v[u][2] : 0.0, in ? (double) v[u][3] : 0.0};
+            } else {
+                *o = in ? (double) v[u][0] : 0.0;
+            }
         }
     };
     for (int64_t c = 0; c < SB_D - 1 && c < chunks; ++c) {
-        f4 v[SB_PER];
+        float v[PER][W];
         load(c, v);
         store(c, v);
     }
@@ -297,41 +369,39 @@ __global__ __launch_bounds__(SB_THREADS) void k_sum_rows_lds(const uint8_t* __re
     double s = 0.0;
     const bool chain = tid < SB_ROWS && r0 + tid < rows;
     for (int64_t c = 0; c < chunks; ++c) {
-        f4 v[SB_PER];
+        float v[PER][W];
         const bool more = c + SB_D - 1 < chunks;
         if (more) load(c + SB_D - 1, v);
         if (chain) {
-            const double* row = ring + (int) (c % SB_D) * SB_ROWS * SB_LD + tid * SB_LD;
-            const int64_t m = n - c * SB_C < SB_C ? n - c * SB_C : SB_C;
-            if (m == SB_C) {
-                // a whole chunk: the next 16 values are read from LDS while the
-                // current 16 are added, so only the adds stay on the chain
-                const sb_d2* row2 = (const sb_d2*) row;
-                sb_d2 cur[8], nxt[8];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) cur[k] = row2[k];
-#pragma unroll
-                for (int g = 0; g < SB_C / 16; ++g) {
-                    if (g + 1 < SB_C / 16) {
-#pragma unroll
-                        for (int k = 0; k < 8; ++k) nxt[k] = row2[8 * (g + 1) + k];
-                    }
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        s = s + cur[k].x;
-                        s = s + cur[k].y;
-                    }
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) cur[k] = nxt[k];
-                }
-            } else {
-                for (int64_t i = 0; i < m; ++i) s = s + row[i];
-            }
+            const int64_t left = n - c * SB_C;
+            s = sum_chain(s, ring + (int) (c % SB_D) * SB_ROWS * SB_LD + tid * SB_LD,
+                          left < SB_C ? ((int) left + 15) / 16 * 16 : SB_C);
         }
         __syncthreads();
         if (more) store(c + SB_D - 1, v);
     }
-    if (chain) part[r0 + tid] = s;
+    // the row sums are written through to where every XCD reads them, then counted
+    if (tid < 64) {
+        if (chain) __hip_atomic_store(part + r0 + tid, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (tid == 0) order = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (order != gridDim.x - 1) return;
+    double total = 0.0;
+    constexpr int BATCH = SB_RING / 16 * 16;
+    for (int64_t b = 0; b < rows; b += BATCH) {
+        const int m = (int) (rows - b < BATCH ? rows - b : BATCH), m16 = (m + 15) / 16 * 16;
+        for (int k = tid; k < m16; k += SB_THREADS)
+            ring[k] = k < m ? __hip_atomic_load(part + b + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+        __syncthreads();
+        if (tid == 0) total = sum_chain(total, ring, m16);
+        __syncthreads();
+    }
+    if (tid == 0) {
+        *d = (float) total;
+        __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+    }
 }
 
 // *d = (float) (0 + part[0] + part[1] + ...), in row order. Up to SC_BATCH row
@@ -420,6 +490,21 @@ __global__ __launch_bounds__(EW_THREADS) void k_acc(const uint8_t* __restrict__ 
             float* t = (float*) (pd + i0 * 4);
             *t = *t + *(const float*) (pb + i0 * sb.nb[0]);
         }
+    }
+}
+
+// k_acc with four floats per lane: rows of b and of the region 16-byte aligned, ne0 a
+// multiple of 4 ([4096, 512]: 7.5 -> 5.5 us; where the region is one run, k_flat does
+// as well)
+__global__ __launch_bounds__(EW_THREADS) void k_acc4(const uint8_t* __restrict__ b, Shape4 sb, uint8_t* __restrict__ d,
+                                                     int64_t offset, int64_t nb1, int64_t nb2, int64_t nb3) {
+    const int64_t rows = sb.ne[1] * sb.ne[2] * sb.ne[3];
+    const int64_t n4 = sb.ne[0] / 4;
+    for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+        const int64_t i1 = r % sb.ne[1], i2 = (r / sb.ne[1]) % sb.ne[2], i3 = r / (sb.ne[1] * sb.ne[2]);
+        const f4* pb = (const f4*) (b + i1 * sb.nb[1] + i2 * sb.nb[2] + i3 * sb.nb[3]);
+        f4* pd = (f4*) (d + offset + i1 * nb1 + i2 * nb2 + i3 * nb3);
+        for (int64_t q = threadIdx.x; q < n4; q += EW_THREADS) pd[q] = pd[q] + pb[q];
     }
 }
 
@@ -565,6 +650,64 @@ __global__ __launch_bounds__(RL_THREADS) void k_repeat_back_lds(const uint8_t* _
     if (tid < 64 && valid) d[j] = s;
 }
 
+// The same sums when ne0 is not repeated and each has few terms (the gradient of a
+// broadcast operand, summed over the planes that shared it): one output, or four
+// along ne0 (VEC: rows of both 16-byte aligned), per lane, RF_AHEAD terms loaded
+// ahead of the in-order adds. Bound by HBM; k_repeat_back_cols asks for 128 terms
+// whatever their number ([64, 333, 12, 2] to 4 planes of the 12: 21.5 -> 4.4 us).
+constexpr int RF_AHEAD = 4;
+template <bool VEC>
+__global__ __launch_bounds__(EW_THREADS) void k_repeat_back_few(const uint8_t* __restrict__ a, Shape4 sa,
+                                                                float* __restrict__ d, uint32_t n, FastDiv ne0,
+                                                                FastDiv ne1, FastDiv ne2, int r1, int r2, int r3) {
+    constexpr int W = VEC ? 4 : 1;
+    const uint32_t j = blockIdx.x * EW_THREADS + threadIdx.x;
+    if (j >= n) return;  // no barrier below
+    const uint32_t q1 = div_by(j, ne0), j0 = j - q1 * ne0.d;
+    const uint32_t q2 = div_by(q1, ne1), j1 = q1 - q2 * ne1.d;
+    const uint32_t j3 = div_by(q2, ne2), j2 = q2 - j3 * ne2.d;
+    const uint8_t* base = a + (int64_t) j0 * W * sa.nb[0] + j1 * sa.nb[1] + j2 * sa.nb[2] + j3 * sa.nb[3];
+    const int64_t st1 = ne1.d * sa.nb[1], st2 = ne2.d * sa.nb[2], st3 = (sa.ne[3] / r3) * sa.nb[3];
+    const int terms = r1 * r2 * r3;
+    // the next term to load, k1 fastest, and its offset
+    int k1 = 0, k2 = 0, k3 = 0, next = 0;
+    auto fetch = [&](float (&v)[W]) {
+        const uint8_t* p = base + (next < terms ? k1 * st1 + k2 * st2 + k3 * st3 : 0);
+        if constexpr (VEC) {
+            const f4 q = *(const f4*) p;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = q[c];
+        } else {
+            v[0] = *(const float*) p;
+        }
+        ++next;
+        if (++k1 == r1) {
+            k1 = 0;
+            if (++k2 == r2) {
+                k2 = 0;
+                ++k3;
+            }
+        }
+    };
+    float s[W];
+#pragma unroll
+    for (int c = 0; c < W; ++c) s[c] = 0.f;
+    for (int t = 0; t < terms; t += RF_AHEAD) {
+        float v[RF_AHEAD][W];
+#pragma unroll
+        for (int u = 0; u < RF_AHEAD; ++u) fetch(v[u]);
+#pragma unroll
+        for (int u = 0; u < RF_AHEAD; ++u) {
+            if (t + u < terms) {  // the same for every lane
+#pragma unroll
+                for (int c = 0; c < W; ++c) s[c] = s[c] + v[u][c];
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < W; ++c) d[(int64_t) j * W + c] = s[c];
+}
+
 unsigned grid_for(int64_t work, int64_t per_block) {
     int64_t g = (work + per_block - 1) / per_block;
     const int64_t cap = (int64_t) device_cus() * 16;
@@ -607,6 +750,23 @@ bool shape_ok(const trc_hip_tensor& t) {
     return true;
 }
 
+bool flat_f32(const trc_hip_tensor& t) { return (((uintptr_t) t.data) & 15u) == 0 && contiguous_f32(t); }
+
+template <FlatOp OP>
+int launch_flat(const char* name, const void* a, const void* b, void* d, int64_t n, float scale, hipStream_t s) {
+    const int64_t blocks = (n / 4 + EW_THREADS) / EW_THREADS;  // one more float4 for the tail
+    if (n >= FLAT_NT) {
+        hipLaunchKernelGGL((k_flat<OP, true>), dim3((unsigned) blocks), dim3(EW_THREADS), 0, s, (const f4*) a,
+                           (const f4*) b, (f4*) d, n, scale);
+    } else {
+        hipLaunchKernelGGL((k_flat<OP, false>), dim3((unsigned) blocks), dim3(EW_THREADS), 0, s, (const f4*) a,
+                           (const f4*) b, (f4*) d, n, scale);
+    }
+    return check_launch(name);
+}
+// grids past one launch's 2^31 workgroups stay with the row kernels
+bool flat_fits(int64_t n) { return n / 4 / EW_THREADS < 0x7FFFFFFF; }
+
 template <BinOp OP>
 int launch_binary(const char* name, const trc_hip_tensor& a, const trc_hip_tensor& b, const trc_hip_tensor& d,
                   hipStream_t s) {
@@ -620,6 +780,9 @@ int launch_binary(const char* name, const trc_hip_tensor& a, const trc_hip_tenso
         }
     }
     if (!f32_aligned(a) || !f32_aligned(b) || !f32_aligned(d)) return fail(TRC_HIP_E_ALIGN, "%s: 4-byte alignment", name);
+    if (flat_f32(a) && flat_f32(d) && flat_f32(b) && nelem(a) == nelem(b) && flat_fits(nelem(d))) {
+        return launch_flat<OP == BinOp::ADD ? FlatOp::ADD : FlatOp::MUL>(name, a.data, b.data, d.data, nelem(d), 0.f, s);
+    }
     const int64_t rows = d.ne[1] * d.ne[2] * d.ne[3];
     if (rows_vec4(a) && rows_vec4(d) && (b.ne[0] == 1 || rows_vec4(b))) {
         hipLaunchKernelGGL(k_binary4<OP>, dim3(grid_for(rows, 1)), dim3(EW_THREADS), 0, s, (const uint8_t*) a.data,
@@ -651,6 +814,9 @@ int launch_unary(const char* name, const trc_hip_tensor& a, const trc_hip_tensor
         if (d.ne[k] != a.ne[k]) return fail(TRC_HIP_E_SHAPE, "%s: dst must have a's shape (dim %d)", name, k);
     }
     if (!f32_aligned(a) || !f32_aligned(d)) return fail(TRC_HIP_E_ALIGN, "%s: 4-byte alignment", name);
+    if (flat_f32(a) && flat_f32(d) && flat_fits(nelem(d))) {
+        return launch_flat<OP == UnOp::SQR ? FlatOp::SQR : FlatOp::SCALE>(name, a.data, nullptr, d.data, nelem(d), scale, s);
+    }
     const int64_t rows = d.ne[1] * d.ne[2] * d.ne[3];
     if (rows_vec4(a) && rows_vec4(d)) {
         hipLaunchKernelGGL(k_unary4<OP>, dim3(grid_for(rows, 1)), dim3(EW_THREADS), 0, s, (const uint8_t*) a.data,
@@ -711,10 +877,19 @@ int launch_sum_f32(const trc_hip_tensor& a, const trc_hip_tensor& d, hipStream_t
     const bool vec = a.nb[0] == 4 && (((uintptr_t) a.data) & 15u) == 0 && (a.ne[1] == 1 || a.nb[1] % 16 == 0) &&
                      (a.ne[2] == 1 || a.nb[2] % 16 == 0) && (a.ne[3] == 1 || a.nb[3] % 16 == 0);
     const unsigned grid = (unsigned) ((rows + SR_THREADS - 1) / SR_THREADS);
-    if (vec && a.ne[0] >= SB_C && a.ne[0] % 4 == 0) {
-        hipLaunchKernelGGL(k_sum_rows_lds, dim3((unsigned) ((rows + SB_ROWS - 1) / SB_ROWS)), dim3(SB_THREADS), 0, s,
-                           (const uint8_t*) a.data, shape_of(a), (double*) ws);
-    } else if (vec) {
+    if (a.ne[0] >= SB_MIN) {
+        uint32_t* ticket = (uint32_t*) (ws + qm_workspace_bytes());
+        const dim3 g((unsigned) ((rows + SB_ROWS - 1) / SB_ROWS));
+        if (vec && a.ne[0] % 4 == 0) {
+            hipLaunchKernelGGL(k_sum_rows_lds<true>, g, dim3(SB_THREADS), 0, s, (const uint8_t*) a.data, shape_of(a),
+                               (double*) ws, ticket, (float*) d.data);
+        } else {
+            hipLaunchKernelGGL(k_sum_rows_lds<false>, g, dim3(SB_THREADS), 0, s, (const uint8_t*) a.data, shape_of(a),
+                               (double*) ws, ticket, (float*) d.data);
+        }
+        return check_launch("sum");
+    }
+    if (vec) {
         hipLaunchKernelGGL(k_sum_rows<true>, dim3(grid), dim3(SR_THREADS), 0, s, (const uint8_t*) a.data, shape_of(a),
                            (double*) ws);
     } else {
@@ -776,6 +951,19 @@ int launch_acc_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const trc_h
         if (rc != TRC_HIP_OK) return rc;
     }
     const int64_t rows = b.ne[1] * b.ne[2] * b.ne[3];
+    // a region as dense as b: one run of floats
+    if (flat_f32(b) && ((((uintptr_t) d.data) | offset) & 15u) == 0 && (b.ne[1] == 1 || nb1 == (size_t) b.ne[0] * 4) &&
+        (b.ne[2] == 1 || nb2 == (size_t) (b.ne[0] * b.ne[1]) * 4) &&
+        (b.ne[3] == 1 || nb3 == (size_t) (b.ne[0] * b.ne[1] * b.ne[2]) * 4) && flat_fits(nelem(b))) {
+        uint8_t* at = (uint8_t*) d.data + offset;
+        return launch_flat<FlatOp::ADD>("acc", at, b.data, at, nelem(b), 0.f, s);
+    }
+    if (rows_vec4(b) && ((((uintptr_t) d.data) | offset) & 15u) == 0 && (b.ne[1] == 1 || nb1 % 16 == 0) &&
+        (b.ne[2] == 1 || nb2 % 16 == 0) && (b.ne[3] == 1 || nb3 % 16 == 0)) {
+        hipLaunchKernelGGL(k_acc4, dim3(grid_for(rows, 1)), dim3(EW_THREADS), 0, s, (const uint8_t*) b.data,
+                           shape_of(b), (uint8_t*) d.data, (int64_t) offset, (int64_t) nb1, (int64_t) nb2, (int64_t) nb3);
+        return check_launch("acc");
+    }
     hipLaunchKernelGGL(k_acc, dim3(grid_for(rows, 1)), dim3(EW_THREADS), 0, s, (const uint8_t*) b.data, shape_of(b),
                        (uint8_t*) d.data, (int64_t) offset, (int64_t) nb1, (int64_t) nb2, (int64_t) nb3);
     return check_launch("acc");
@@ -795,6 +983,24 @@ int launch_repeat_back_f32(const trc_hip_tensor& a, const trc_hip_tensor& d, hip
     if (a.ne[0] == d.ne[0] && a.ne[2] == d.ne[2] && a.ne[3] == d.ne[3] && a.ne[1] / d.ne[1] >= 2 * RL_T) {
         hipLaunchKernelGGL(k_repeat_back_lds, dim3((unsigned) ((n + 63) / 64)), dim3(RL_THREADS), 0, s,
                            (const uint8_t*) a.data, shape_of(a), (float*) d.data, shape_of(d));
+        return check_launch("repeat_back");
+    }
+    const int64_t r1 = a.ne[1] / d.ne[1], r2 = a.ne[2] / d.ne[2], r3 = a.ne[3] / d.ne[3];
+    // up to RB_AHEAD terms: more keep the pipeline of k_repeat_back_cols busy
+    if (a.ne[0] == d.ne[0] && r1 <= RB_AHEAD && r2 <= RB_AHEAD && r3 <= RB_AHEAD && r1 * r2 * r3 <= RB_AHEAD &&
+        n < ((int64_t) 1 << 31) - EW_THREADS) {
+        const bool vec = rows_vec4(a) && (((uintptr_t) d.data) & 15u) == 0;
+        const int64_t units = vec ? n / 4 : n, u0 = vec ? d.ne[0] / 4 : d.ne[0];
+        const dim3 grid((unsigned) ((units + EW_THREADS - 1) / EW_THREADS));
+        if (vec) {
+            hipLaunchKernelGGL(k_repeat_back_few<true>, grid, dim3(EW_THREADS), 0, s, (const uint8_t*) a.data, shape_of(a),
+                               (float*) d.data, (uint32_t) units, fast_div(u0), fast_div(d.ne[1]), fast_div(d.ne[2]),
+                               (int) r1, (int) r2, (int) r3);
+        } else {
+            hipLaunchKernelGGL(k_repeat_back_few<false>, grid, dim3(EW_THREADS), 0, s, (const uint8_t*) a.data, shape_of(a),
+                               (float*) d.data, (uint32_t) units, fast_div(u0), fast_div(d.ne[1]), fast_div(d.ne[2]),
+                               (int) r1, (int) r2, (int) r3);
+        }
         return check_launch("repeat_back");
     }
     if (a.ne[0] == d.ne[0]) {
