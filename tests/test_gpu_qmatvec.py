@@ -454,3 +454,32 @@ def test_random_routes(hip, name, K, M, N, x_pad, y_pad):
     got = gpu_qmatvec(t, raw, K, M, X, x_pad=x_pad, y_pad=y_pad)
     want = oracle_qmatvec(t, raw, K, M, X)
     assert O.row_l2_error(got, want) <= TOL
+
+
+@pytest.mark.parametrize("name", list(TYPES))
+@pytest.mark.parametrize("K,M,N", [(256, 70, 33), (4096, 300, 49), (4096, 2100, 64), (1536, 8193, 49), (512, 9000, 48),
+                                   (32768, 40, 50), (33024, 40, 50)])
+def test_two_slices_of_columns(hip, name, K, M, N):
+    """33 to 64 columns: two slices of 32 in one call (the second from 1 to 32 columns
+    wide, K whole and in two parts, up to the longest K whose x the workspace holds
+    twice), and beyond those limits one call per slice. Against float64 (the oracle's
+    own float sums are off by sqrt(K) half ulps, 3e-6 at K = 32768): x is held to 22
+    bits and the sums of blocks are FP32, so the row-L2 error is a few 2^-22."""
+    announce(f"qmatvec two slices {name} K={K} M={M} N={N}")
+    t = TYPES[name]
+    raw = synth.block_bytes(synth.quant_blocks(t, K * M // 32, 970 + K))
+    X = synth.normal(971 + N, K * N).reshape(1, 1, N, K)
+    dw, dx, dy = Dev(raw), Dev(X), empty((1, 1, N, M))
+    args = (t, dw.ptr, K, M, (K // 32) * H.BLOCK_BYTES[t], dx.ptr, N, K * 4, dy.ptr, M * 4)
+    H.fill_f32(dy.ptr, float("nan"), N * M)
+    H.qmatvec(*args)
+    H.sync()
+    got = dy.read().copy()
+    W = O.dequant(t, raw, threads=8).reshape(M, K).astype(np.float64)
+    want = X.astype(np.float64) @ W.T
+    assert (np.abs(got - want).max(-1) / np.linalg.norm(want, axis=-1)).max() <= 1e-6
+    H.qmatvec_noalloc(*args)
+    H.sync()
+    assert np.array_equal(dy.read().view(np.uint32), got.view(np.uint32))
+    for d in (dw, dx, dy):
+        d.free()

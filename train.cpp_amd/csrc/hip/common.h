@@ -133,8 +133,8 @@ int launch_mul_mat_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const t
 enum class QmScratch { PER_STREAM, STATIC };
 int launch_qmatvec(int type, const void* wq, int64_t K, int64_t M, size_t nb1_w, const float* x,
                    int64_t N, size_t nb1_x, float* y, size_t nb1_y, hipStream_t stream, QmScratch where);
-// Fused quant x skinny GEMM on the fp16 matrix cores for 2 <= N <= 32 (N = 2, 3
-// only off the integer-dot kernel's alignment)
+// Fused quant x skinny GEMM on the fp16 matrix cores for 2 <= N <= 64 (N = 2, 3
+// only off the integer-dot kernel's alignment; over 32 with K <= 32768)
 // (qmm.hip); qmm_supported says whether the shape and alignment fit it.
 bool qmm_supported(int64_t K, int64_t N, const void* wq, size_t nb1_w);
 int launch_qmm(int type, const void* wq, int64_t K, int64_t M, size_t nb1_w, const float* x, int64_t N,

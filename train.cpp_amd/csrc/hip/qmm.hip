@@ -1,7 +1,9 @@
-// H2 for 2 <= N <= 32 columns: fused dequant x skinny GEMM on the fp16 matrix
-// cores (v_mfma_f32_16x16x32_f16). Columns come in tiles of 16; one launch
+// H2 for 2 <= N <= 64 columns: fused dequant x skinny GEMM on the fp16 matrix
+// cores (v_mfma_f32_16x16x32_f16). Columns come in tiles of 16; a workgroup
 // carries one or two tiles (NT), so every weight is read and decoded once per
-// 32 columns.
+// 32 columns, and over 32 columns two slices of 32 run side by side in one launch:
+// bound by the x operands every workgroup reads from L2, they take twice the rows
+// per workgroup (K = 11008, M = 4096, N = 50 41.0 -> 27.6 us, N = 64 41.4 -> 28.6).
 //
 // Result to reproduce: gguf_tensor_to_f32 (src/io/trc_gguf.cpp:966-1049,
 // dequantize_q* :320-417) followed by compute_mul_mat
@@ -88,6 +90,11 @@ constexpr uint32_t QM_RSRC_WORD3 = 0x00020000u;  // gfx9 buffer resource: raw 32
 constexpr int QM_A_BYTES = QM_NT * QM_MAX_BLOCKS * 2 * 64 * 16;
 constexpr int QM_META_BYTES = (QM_META_XS + QM_MAX_BLOCKS * QM_COLS) * 4;
 static_assert(QM_A_BYTES % 256 == 0, "the meta floats start 256-byte aligned");
+
+// Two slices of 32 columns (33 <= N <= 64) in one call: the second's blocks follow
+// QM_SLICE blocks after the first's in every array of the workspace, so half the K.
+constexpr int QM_SLICE = QM_MAX_BLOCKS / 2;
+static_assert(QM_SLICE % QM_CHB == 0, "a slice starts at a chunk");
 
 template <int TYPE>
 constexpr bool rotated_even() {
@@ -193,31 +200,37 @@ __device__ __forceinline__ QmXConv qm_xconv(const float2 (&w)[4]) {
 // A launch split over K adds two partial sums into y, so then (y0 != nullptr)
 // the wave also clears its share of column j of y: rows
 // [ch * per, (ch + 1) * per) with per = ceil(M / chunks).
+template <bool SLICES>
 __global__ __launch_bounds__(64) void k_qmm_xprep(const float* __restrict__ x, int64_t ldx, int N, int nblk, int rot,
                                                    int ncol, int pk, float* __restrict__ y0, int64_t ldy, int64_t M,
                                                    uint8_t* __restrict__ ws) {
     uint4* const xa = (uint4*) ws;
     float* const meta = (float*) (ws + QM_A_BYTES);
     const int ch = blockIdx.x / ncol, j = blockIdx.x % ncol;  // columns past N get zeros
+    const int slice = SLICES ? blockIdx.y : 0;
+    x += (int64_t) slice * QM_COLS * ldx;
+    N -= slice * QM_COLS;
     const int l = threadIdx.x, bl = l >> 2, g = l & 3;
     if (y0 != nullptr && j < N) {
         const int64_t nchunks = gridDim.x / ncol, per = (M + nchunks - 1) / nchunks;
         const int64_t a = ch * per, e = a + per < M ? a + per : M;
-        for (int64_t m = a + l; m < e; m += 64) y0[j * ldy + m] = 0.f;
+        for (int64_t m = a + l; m < e; m += 64) y0[(slice * QM_COLS + j) * ldy + m] = 0.f;
     }
     float2 v[4];
     qm_xload(x, ldx, N, nblk, rot, ch, j, l, v);
     const QmXConv r = qm_xconv(v);
     const int b = ch * QM_CHB + bl;
     if (b < nblk) {
-        uint4* dst = xa + ((int64_t) (j >> 4) * QM_MAX_BLOCKS + b) * 2 * 64 + (j & 15) + 16 * g;
+        const int sb = slice * QM_SLICE + b;
+        uint4* dst = xa + ((int64_t) (j >> 4) * QM_MAX_BLOCKS + sb) * 2 * 64 + (j & 15) + 16 * g;
         dst[0] = __builtin_bit_cast(uint4, r.hi);
         dst[pk ? 8 : 64] = __builtin_bit_cast(uint4, r.lo);
-        if (g == 0) meta[QM_META_XS + b * QM_COLS + j] = r.sm;
-        if (pk && g == 0) meta[QM_META_XS + b * QM_COLS + j + 8] = 0.f;
+        if (g == 0) meta[QM_META_XS + sb * QM_COLS + j] = r.sm;
+        if (pk && g == 0) meta[QM_META_XS + sb * QM_COLS + j + 8] = 0.f;
     }
-    if (l == 0) meta[ch * QM_COLS + j] = r.sc;
-    if (pk && l == 0) meta[ch * QM_COLS + j + 8] = r.sc;
+    const int sch = slice * (QM_SLICE / QM_CHB) + ch;
+    if (l == 0) meta[sch * QM_COLS + j] = r.sc;
+    if (pk && l == 0) meta[sch * QM_COLS + j + 8] = r.sc;
 }
 
 // Per format: which dwords of a pair each lane loads (NW of them), in bytes
@@ -574,6 +587,13 @@ __global__ __launch_bounds__(QM_WAVES * 64) void k_qmm(const uint8_t* __restrict
     const int c0 = blockIdx.y * part_chunks;                             // this part's first chunk
     const int nl = part_chunks < nch - c0 ? part_chunks : nch - c0;      // and its chunk count (>= 1)
     const uint32_t sel = g < 3 ? 0x03020100u : 0x03020504u;
+    // the slice of 32 columns
+    int xpair0 = 0;
+    if constexpr (NT == 2) {
+        y += (int64_t) blockIdx.z * QM_COLS * ldy;
+        N -= (int) blockIdx.z * QM_COLS;
+        xpair0 = (int) blockIdx.z * (QM_SLICE / 2);
+    }
 
     // The workgroup's rows as one buffer (the launcher keeps it below 2^31 bytes).
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
@@ -630,7 +650,7 @@ __global__ __launch_bounds__(QM_WAVES * 64) void k_qmm(const uint8_t* __restrict
     // x operands of this wave's pair of the part's chunk c -> xr[xs]
     auto load_x = [&](int c, int xs) {
         const int p = (c0 + (c < nl ? c : nl - 1)) * QM_CP + wave;
-        qm_load_x<TYPE, NT, PK>(xr[xs], rx, rm, xo, mo, p < np ? p : np - 1);
+        qm_load_x<TYPE, NT, PK>(xr[xs], rx, rm, xo, mo, xpair0 + (p < np ? p : np - 1));
     };
     // Step c. Loads go out per chunk as W then x, so once at most (R - 1) chunks'
     // loads are outstanding, chunk c's W (this wave's part) and x have landed;
@@ -769,7 +789,7 @@ struct QmCall {
     float* y;
     size_t nb1_y;
     int N;
-    int rows, parts, part_chunks;
+    int rows, parts, part_chunks, slices;
     const uint8_t* ws;
     const float* x;  // read by the kernel only when it converts x itself
     size_t nb1_x;
@@ -783,7 +803,7 @@ int launch_t(const QmCall& q) {
         return fail(TRC_HIP_E_INVALID, "qmm: %d rows per workgroup and x exceed the LDS", q.rows);
     } else {
         const int64_t grid = (q.M + q.rows - 1) / q.rows;
-        hipLaunchKernelGGL((k_qmm<TYPE, T, ROUNDS, R, NT, PK, LXC>), dim3((unsigned) grid, (unsigned) q.parts),
+        hipLaunchKernelGGL((k_qmm<TYPE, T, ROUNDS, R, NT, PK, LXC>), dim3((unsigned) grid, (unsigned) q.parts, (unsigned) q.slices),
                            dim3(QM_WAVES * 64), 0, q.s, (const uint8_t*) q.wq, q.nblk, q.M, (int64_t) q.nb1_w, q.y,
                            (int64_t) (q.nb1_y / sizeof(float)), q.N, q.rows, q.part_chunks, q.ws, q.x,
                            (int64_t) (q.nb1_x / sizeof(float)));
@@ -863,17 +883,20 @@ int launch_tiles(int t, const QmCall& q) {
 struct QmPlan {
     int rows, parts, part_chunks;
 };
+// Two slices count as twice the rows, and their x operands (64 KB a chunk, whatever
+// the rows) weigh more: K is split up to the largest row count instead (K = 11008,
+// M = 4096, N = 50: a chunk takes 1.35 us with 32 rows, 2.0 with 64).
 template <int TYPE, int NT>
-QmPlan qm_plan(int nblk, int64_t M) {
+QmPlan qm_plan(int nblk, int64_t M, int slices) {
     const int nch = (nblk / 2 + QM_CP - 1) / QM_CP;
     const int64_t cus = device_cus();
     QmPlan p;
     // measured at K = 4096, N = 8 and 16: the split is faster from M = 2048
     // (-15 %) to 6144 (-1 %), slower from 8192
-    p.parts = nch >= 2 && (M + cus - 1) / cus <= 24 ? 2 : 1;
+    p.parts = nch >= 2 && (slices == 2 ? 4 * M <= qm_max_rows<TYPE, NT>() * cus : (M + cus - 1) / cus <= 24) ? 2 : 1;
     p.part_chunks = (nch + p.parts - 1) / p.parts;
     p.parts = (nch + p.part_chunks - 1) / p.part_chunks;
-    int64_t rows = (M * p.parts + cus - 1) / cus;
+    int64_t rows = (M * p.parts * slices + cus - 1) / cus;
     rows = (rows + 7) / 8 * 8;
     if (rows > qm_max_rows<TYPE, NT>()) rows = qm_max_rows<TYPE, NT>();
     p.rows = (int) rows;
@@ -913,27 +936,31 @@ bool qm_lx_fits(const QmPlan& p) {
     }
 }
 
-// NT = 1 for N <= 16, 2 for 17 <= N <= 32: every column tile shares one pass over W.
+// NT = 1 for N <= 16, 2 for 17 <= N <= 64: the column tiles of 32 columns share one
+// pass over W; beyond 32 two slices of 32 run in one launch each of the pre-pass and
+// the product.
 // PK (N <= 8): x hi and lo packed into one tile; with K in one part whose x fits
 // beside the ring, each workgroup converts x itself and no pre-pass runs.
 template <int TYPE, int NT, bool PK>
 int launch_fmt(const void* wq, int nblk, int64_t M, size_t nb1_w, const float* x, size_t nb1_x, int N, float* y,
                size_t nb1_y, QmScratch where, hipStream_t s) {
-    const QmPlan p = qm_plan<TYPE, NT>(nblk, M);
+    const int slices = (N + QM_COLS - 1) / QM_COLS;
+    const QmPlan p = qm_plan<TYPE, NT>(nblk, M, slices);
     const int tiles = (p.rows + 15) / 16;
     if constexpr (PK) {
         if (qm_lx_fits<TYPE>(p)) {  // x converted in the kernel: no workspace
-            const QmCall q{wq, nblk, M, nb1_w, y, nb1_y, N, p.rows, p.parts, p.part_chunks, nullptr, x, nb1_x, s};
+            const QmCall q{wq, nblk, M, nb1_w, y, nb1_y, N, p.rows, p.parts, p.part_chunks, 1, nullptr, x, nb1_x, s};
             return launch_tiles<TYPE, 1, NT, PK, QM_LXC>(tiles, q);
         }
     }
     uint8_t* ws = nullptr;
     const int wrc = where == QmScratch::STATIC ? qm_static_scratch(&ws) : qm_stream_workspace(s, &ws);
     if (wrc != TRC_HIP_OK) return wrc;
-    const QmCall q{wq, nblk, M, nb1_w, y, nb1_y, N, p.rows, p.parts, p.part_chunks, ws, x, nb1_x, s};
+    const QmCall q{wq, nblk, M, nb1_w, y, nb1_y, N, p.rows, p.parts, p.part_chunks, slices, ws, x, nb1_x, s};
     const int nchunks = (nblk + QM_CHB - 1) / QM_CHB;
     const int ncol = PK ? 8 : 16 * NT;  // one pre-pass wave per chunk and column
-    hipLaunchKernelGGL(k_qmm_xprep, dim3((unsigned) (nchunks * ncol)), dim3(64), 0, s, x,
+    auto* const prep = slices > 1 ? k_qmm_xprep<true> : k_qmm_xprep<false>;
+    hipLaunchKernelGGL(prep, dim3((unsigned) (nchunks * ncol), (unsigned) slices), dim3(64), 0, s, x,
                        (int64_t) (nb1_x / sizeof(float)), N, nblk, rotated_even<TYPE>() ? 2 : 0, ncol, PK ? 1 : 0,
                        p.parts > 1 ? y : nullptr, (int64_t) (nb1_y / sizeof(float)), M, ws);
     const int rc = check_launch("qmm_xprep");
@@ -956,7 +983,8 @@ bool qmm_supported(int64_t K, int64_t N, const void* wq, size_t nb1_w) {
     // K chunks are copied in 16-byte pieces (a multiple of 4 pairs per row keeps them
     // aligned); a workgroup's rows (at most 112) are addressed through one buffer
     // resource (< 2^31 bytes)
-    return N >= 2 && N <= 16 * QM_NT && nblk >= 8 && nblk % 8 == 0 && nblk <= QM_MAX_BLOCKS &&
+    // (two slices of columns share the x workspace: half the K)
+    return N >= 2 && N <= (nblk <= QM_SLICE ? 2 : 1) * QM_COLS && nblk >= 8 && nblk % 8 == 0 && nblk <= QM_MAX_BLOCKS &&
            (((uintptr_t) wq) & 15u) == 0 && (nb1_w & 15u) == 0 && nb1_w <= ((size_t) 1 << 24);
 }
 
