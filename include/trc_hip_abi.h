@@ -267,9 +267,10 @@ int trc_hip_scale_f32(const trc_hip_tensor* a, const trc_hip_tensor* dst, float 
  * OP_SUM (src/ops/trc_ops.cpp:214-221) as computed by compute_sum
  * (src/backends/cpu/trc_cpu_ops.cpp:302-315, row_sum_f32 :284-300): each row
  * (ne0-run) is summed in double from 0 in element order, the row sums are added
- * in double in row order, and the total is rounded to float once; the same
- * operations in the same order, so the result is bit-identical. Rows are summed
- * in parallel (each row's own sum stays sequential) into the stream's x
+ * in double in row order, and the total is rounded to float once; the result is
+ * bit-identical: the same operations in the same order (rows in parallel, each
+ * row's own sum sequential), or, for long contiguous data, a sum in another order
+ * whose error bound shows that both round to the same float. It uses the stream's x
  * workspace of trc_hip_qmatvec, which the first such call on a stream allocates
  * (make it before capturing that stream in global mode); more rows than that
  * workspace holds (about a million) are summed by one workgroup. */

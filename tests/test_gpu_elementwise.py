@@ -394,6 +394,58 @@ def test_sum_staged_rows_bitwise(hip, shape, cut):
     assert bits(gpu_sum(t, np.swapaxes(t, -1, -2)[..., :av.shape[-1]])) == want
 
 
+def sum_case(shape, kind, rng):
+    """Data whose sum in any order settles the result (squares), whose order shows
+    (cancelling, a tie between two floats), or that is not finite."""
+    a = rng.standard_normal(shape).astype(np.float32)
+    f = a.reshape(-1)
+    if kind == "squares":
+        a *= a
+    elif kind == "cancel":  # 2^53 swallows what follows it until it is taken off again
+        f *= np.float32(2.0 ** -2)
+        f[1::97] = np.float32(2.0 ** 53)
+        f[60::97] = -np.float32(2.0 ** 53)
+    elif kind in ("tie", "above"):
+        f[:] = 0
+        f[f.size // 3], f[f.size // 2] = 1, 2.0 ** -24
+        if kind == "above":  # past the tie by 2^-50, or not, by the order of the first rounding
+            f[-1] = 2.0 ** -50
+    elif kind == "inf":
+        f[-1] = np.inf
+    elif kind == "nan":
+        f[f.size // 2] = np.nan
+    elif kind == "huge":
+        f[:] = 3e38
+    elif kind == "minus zero":
+        f[:] = -0.0
+    elif kind == "subnormal":
+        f *= np.float32(1e-41)
+    return a
+
+
+@pytest.mark.parametrize("kind", ["squares", "normal", "cancel", "tie", "above", "inf", "nan", "huge", "minus zero",
+                                  "subnormal"])
+@pytest.mark.parametrize("shape,off", [((1, 511), 0), ((1, 512), 1), ((447, 64), 0), ((448, 64), 0), ((130, 777), 3),
+                                       ((64, 4096), 0), ((2, 2_100_001), 2), ((3, 5, 40, 1000), 1)])
+def test_sum_any_order_bitwise(hip, shape, off, kind):
+    """Contiguous operands summed in any order first: both sides of the size from
+    which that is done, bases at every place within 16 bytes, one and several
+    floats per thread; the bits are those of the sum in order whatever the data."""
+    announce(f"sum any order {shape} off {off} {kind}")
+    rng = np.random.default_rng(29)
+    a = sum_case(shape, kind, rng)
+    base = np.zeros(a.size + off, np.float32)
+    base[off:] = a.reshape(-1)
+    view = base[off:].reshape(shape)
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = bits(O.sum_all(view))
+    got = [gpu_sum(base, view) for _ in range(2)]
+    if kind == "nan":
+        assert all(np.isnan(g) for g in got)
+    else:
+        assert [bits(g) for g in got] == [want, want]
+
+
 @pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1024, 1027, 100_001])
 @pytest.mark.parametrize("off", [0, 1])
 def test_contiguous_elementwise_bitwise(hip, n, off):

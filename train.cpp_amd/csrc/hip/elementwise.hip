@@ -200,7 +200,8 @@ __global__ __launch_bounds__(EW_THREADS) void k_repeat(const uint8_t* __restrict
 // fastest, then i2, i3), one rounding to float at the end.
 //
 // Rows of 64 elements and more (k_sum_rows_lds) stream through LDS and meet in the
-// workgroup that finishes last. Shorter rows take two launches: k_sum_rows, one
+// workgroup that finishes last, unless the sum in any order settles the result
+// (k_sum_bounded below). Shorter rows take two launches: k_sum_rows, one
 // lane per row with the row's next SR_AHEAD loads issued ahead of the adds (from
 // addresses clamped into the row, so no branch waits on them), then k_sum_combine,
 // one wave that adds the row sums in row order. k_sum (one workgroup, no
@@ -271,6 +272,7 @@ __global__ __launch_bounds__(SR_THREADS) void k_sum_rows(const uint8_t* __restri
 // per row, 13 here.
 // The workgroup that takes the last ticket adds the row sums in row order (512
 // rows of 4096 40.0 us with a launch of its own for that, 37.2 here).
+// CHECKED: runs behind k_sum_bounded, whose sums may make all of this unnecessary.
 constexpr int SB_ROWS = 8;
 constexpr int SB_THREADS = 256;
 constexpr int SB_C = 256;
@@ -306,15 +308,122 @@ __device__ __forceinline__ double sum_chain(double s, const double* p, int n) {
     return s;
 }
 
-template <bool VEC>
+// The chain above is what the order of the sum costs, and mostly the order does not
+// matter: one pass over contiguous data gives S, its sum in double in some order, and
+// A, the sum of the magnitudes. With u = 2^-53 and at most k roundings on an
+// element's way into either sum, both lie within k u A (1 + k u) of the true sum (N.
+// J. Higham, "Accuracy and Stability of Numerical Algorithms", 4.2), so the sum in
+// the stated order lies within b of S, b = 1.01 u A times the k of both orders and a
+// few for the check's own roundings. Rounding to float is monotone: where S - b and
+// S + b round to the same float, so does the sum in order, and that float is its
+// result bit for bit. Elsewhere (A not finite, or S within b of the middle of two
+// floats: about k u A / (6e-8 |S|) of all sums, 2e-5 of the sums of 512 x 4096
+// squares) the chain runs as without this.
+// S and A stay one pair per workgroup; every workgroup of the second launch adds
+// the pairs up in one order and comes to the same decision, so that no ticket, flag
+// or wait lies between. Bound by two launches, then by HBM (65536 x 4096 5.6 TB/s).
+// Chain -> here, both launches: [777, 130] 13.0 -> 6.7 us, [4096, 512] 37.2 -> 6.8,
+// [333, 7992 rows] 68.5 -> 7.5, [4096, 65536] 954 -> 191; where the chain has to run
+// all the same, 4.5 us more.
+constexpr int SUMB_THREADS = 1024;
+constexpr int SUMB_MAX = SB_THREADS;  // workgroups: a pair for each thread of the second launch
+constexpr int SUMB_V = 4;             // float4s in flight per thread
+// row length + rows (the length of the chain) from which on the pass and its launch
+// pay for themselves: 16 x 400 6.6 us both ways, 128 x 256 6.7 -> 6.9, 256 x 256 7.4 ->
+// 6.7, 16 x 512 7.3 -> 6.7
+constexpr int SUMB_MIN = 512;
+struct SumPair {
+    double s, a;
+};
+constexpr size_t SUMB_BYTES = SUMB_MAX * sizeof(SumPair);
+
+// the pair of all WAVES waves' lanes, in every thread (sh: one pair per wave)
+template <int WAVES>
+__device__ __forceinline__ SumPair sum_pair_all(SumPair v, SumPair* sh) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        v.s += __shfl_xor(v.s, o);
+        v.a += __shfl_xor(v.a, o);
+    }
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    SumPair t = sh[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) {
+        t.s += sh[w].s;
+        t.a += sh[w].a;
+    }
+    __syncthreads();
+    return t;
+}
+
+// pairs[workgroup] = the sum and the sum of magnitudes of its share of n floats. The
+// float4s begin at the first 16-byte boundary; what lies before and after them goes
+// to the first threads of workgroup 0.
+__global__ __launch_bounds__(SUMB_THREADS) void k_sum_bounded(const float* __restrict__ a, int64_t n,
+                                                              SumPair* __restrict__ pairs) {
+    __shared__ SumPair sh[SUMB_THREADS / 64];
+    const int64_t pre = (int64_t) ((16u - (uint32_t) ((uintptr_t) a & 15u)) & 15u) / 4;
+    const int64_t head = pre < n ? pre : n;
+    const int64_t n4 = (n - head) / 4;
+    const f4* v = (const f4*) (a + head);
+    double s[4] = {0.0, 0.0, 0.0, 0.0}, m[4] = {0.0, 0.0, 0.0, 0.0};
+    auto add = [&](int k, float x) {
+        const double e = (double) x;
+        s[k] += e;
+        m[k] += __builtin_fabs(e);
+    };
+    const int64_t stride = (int64_t) gridDim.x * SUMB_THREADS;
+    int64_t i = (int64_t) blockIdx.x * SUMB_THREADS + threadIdx.x;
+    for (; i + (SUMB_V - 1) * stride < n4; i += SUMB_V * stride) {
+        f4 q[SUMB_V];
+#pragma unroll
+        for (int u = 0; u < SUMB_V; ++u) q[u] = v[i + u * stride];
+#pragma unroll
+        for (int u = 0; u < SUMB_V; ++u)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) add(k, q[u][k]);
+    }
+    for (; i < n4; i += stride) {
+        const f4 q = v[i];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) add(k, q[k]);
+    }
+    if (blockIdx.x == 0) {
+        const int64_t rest = n - head - 4 * n4;  // under 4, as head is
+        if ((int64_t) threadIdx.x < head) add(0, a[threadIdx.x]);
+        if ((int64_t) threadIdx.x < rest) add(1, a[head + 4 * n4 + threadIdx.x]);
+    }
+    const SumPair t = sum_pair_all<SUMB_THREADS / 64>({(s[0] + s[1]) + (s[2] + s[3]), (m[0] + m[1]) + (m[2] + m[3])}, sh);
+    if (threadIdx.x == 0) pairs[blockIdx.x] = t;
+}
+
+struct SumCheck {
+    const SumPair* pairs;
+    int n;         // of them
+    double rel;    // b / A
+};
+
+template <bool VEC, bool CHECKED>
 __global__ __launch_bounds__(SB_THREADS) void k_sum_rows_lds(const uint8_t* __restrict__ a, Shape4 sa, double* part,
-                                                             uint32_t* ticket, float* __restrict__ d) {
+                                                             uint32_t* ticket, float* __restrict__ d, SumCheck chk) {
     constexpr int W = VEC ? 4 : 1;                         // elements per load
     constexpr int PER = SB_ROWS * SB_C / W / SB_THREADS;   // loads per thread and chunk
     static_assert(PER * SB_THREADS * W == SB_ROWS * SB_C, "a chunk is whole loads per thread");
     static_assert(SB_C / W <= SB_THREADS, "a thread's loads are whole rows apart");
     __shared__ __attribute__((aligned(16))) double ring[SB_RING];
     __shared__ uint32_t order;
+    if constexpr (CHECKED) {
+        SumPair v = {0.0, 0.0};
+        if ((int) threadIdx.x < chk.n) v = chk.pairs[threadIdx.x];
+        v = sum_pair_all<SB_THREADS / 64>(v, (SumPair*) ring);
+        const double b = chk.rel * v.a;
+        const float lo = (float) (v.s - b), hi = (float) (v.s + b);
+        if (v.a < __builtin_inf() && __builtin_bit_cast(uint32_t, lo) == __builtin_bit_cast(uint32_t, hi)) {
+            if (blockIdx.x == 0 && threadIdx.x == 0) *d = lo;
+            return;
+        }
+    }
     const int64_t rows = sa.ne[1] * sa.ne[2] * sa.ne[3];
     const int64_t r0 = (int64_t) blockIdx.x * SB_ROWS;
     const int64_t n = sa.ne[0];
@@ -880,13 +989,37 @@ int launch_sum_f32(const trc_hip_tensor& a, const trc_hip_tensor& d, hipStream_t
     if (a.ne[0] >= SB_MIN) {
         uint32_t* ticket = (uint32_t*) (ws + qm_workspace_bytes());
         const dim3 g((unsigned) ((rows + SB_ROWS - 1) / SB_ROWS));
-        if (vec && a.ne[0] % 4 == 0) {
-            hipLaunchKernelGGL(k_sum_rows_lds<true>, g, dim3(SB_THREADS), 0, s, (const uint8_t*) a.data, shape_of(a),
-                               (double*) ws, ticket, (float*) d.data);
-        } else {
-            hipLaunchKernelGGL(k_sum_rows_lds<false>, g, dim3(SB_THREADS), 0, s, (const uint8_t*) a.data, shape_of(a),
-                               (double*) ws, ticket, (float*) d.data);
+        const bool whole = vec && a.ne[0] % 4 == 0;
+        const int64_t n = rows * a.ne[0];
+        const bool run = a.nb[0] == 4 && (a.ne[1] == 1 || (int64_t) a.nb[1] == 4 * a.ne[0]) &&
+                         (a.ne[2] == 1 || (int64_t) a.nb[2] == 4 * a.ne[0] * a.ne[1]) &&
+                         (a.ne[3] == 1 || (int64_t) a.nb[3] == 4 * a.ne[0] * a.ne[1] * a.ne[2]);
+        SumCheck chk = {nullptr, 0, 0.0};
+        if (run && a.ne[0] + rows >= SUMB_MIN && (size_t) rows * sizeof(double) + SUMB_BYTES <= qm_workspace_bytes()) {
+            SumPair* pairs = (SumPair*) (ws + qm_workspace_bytes() - SUMB_BYTES);
+            const int64_t want = (n + 4 * SUMB_THREADS - 1) / (4 * SUMB_THREADS);
+            chk.pairs = pairs;
+            chk.n = (int) (want < SUMB_MAX ? want : SUMB_MAX);
+            // roundings on the way of an element: the rows and the row sums; here a
+            // thread's, a workgroup's (2 + 6 + 15) and the pairs' (6 + 3); the check's
+            const double k = (double) a.ne[0] + (double) rows + (double) n / ((double) chk.n * SUMB_THREADS) + 64.0;
+            chk.rel = 1.01 * k * 0x1p-53;
+            hipLaunchKernelGGL(k_sum_bounded, dim3((unsigned) chk.n), dim3(SUMB_THREADS), 0, s, (const float*) a.data, n,
+                               pairs);
+            const int st = check_launch("sum (in any order)");
+            if (st != TRC_HIP_OK) return st;
         }
+#define TRC_SUM(V, C)                                                                                              \
+    hipLaunchKernelGGL((k_sum_rows_lds<V, C>), g, dim3(SB_THREADS), 0, s, (const uint8_t*) a.data, shape_of(a), \
+                       (double*) ws, ticket, (float*) d.data, chk)
+        if (whole) {
+            if (chk.n) TRC_SUM(true, true);
+            else TRC_SUM(true, false);
+        } else {
+            if (chk.n) TRC_SUM(false, true);
+            else TRC_SUM(false, false);
+        }
+#undef TRC_SUM
         return check_launch("sum");
     }
     if (vec) {
