@@ -1518,7 +1518,7 @@ int launch_qmatvec(int type, const void* wq, int64_t K, int64_t M, size_t nb1_w,
     // for 32 columns and a narrower one for the rest take less (Q4_0, K = 4096, M =
     // 14336, one call against two: N = 33 33.8 / 28.4 us, 40 33.3 / 32.3, 48 33.5 /
     // 33.6, 64 33.8 / 39.0; K = 11008, M = 4096: N = 33 27.3 / 31.2, 50 27.6 / 41.0).
-    const bool slices = N > 48 || M <= 32 * (int64_t) device_cus();
+    const bool slices = N > 48 || (N > 32 && M <= 32 * (int64_t) device_cus());
     if (N > 16 && !((N <= 32 || slices) && qmm_supported(K, N, wq, nb1_w))) {
         // skinny GEMM beyond the columns one launch carries: one fused pass over W
         // per 32 columns on the matrix-core kernel, else per 16 (the launches run
