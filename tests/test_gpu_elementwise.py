@@ -446,6 +446,23 @@ def test_sum_any_order_bitwise(hip, shape, off, kind):
         assert [bits(g) for g in got] == [want, want]
 
 
+@pytest.mark.parametrize("n", [1, 16, 17, 777, 8192, 8193])
+@pytest.mark.parametrize("terms", [64, 127, 128, 129, 256, 257, 700])
+def test_repeat_back_staged_terms_bitwise(hip, n, terms):
+    """Terms at the edges of a chunk of 128 and of the ring's first chunks, outputs at
+    the edges of 16 a workgroup and of the size from which on it takes 64."""
+    announce(f"repeat_back staged n {n} terms {terms}")
+    rng = np.random.default_rng(30)
+    a = rng.standard_normal((terms, n)).astype(np.float32)
+    da, out = Dev(a), empty((n,))
+    H.repeat_back_f32(da.tensor(), out.tensor())
+    H.sync()
+    got = out.read()
+    da.free()
+    out.free()
+    assert (bits(got).ravel() == bits(O.repeat_back(a, [n, 1, 1, 1])).ravel()).all()
+
+
 @pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1024, 1027, 100_001])
 @pytest.mark.parametrize("off", [0, 1])
 def test_contiguous_elementwise_bitwise(hip, n, off):

@@ -695,20 +695,29 @@ __global__ __launch_bounds__(RB_THREADS) void k_repeat_back_cols(const uint8_t* 
 }
 
 // k_repeat_back_cols when only dim 1 repeats (output j's terms are a's element j
-// and every st1 bytes after it), with the loads spread over a workgroup: 64
-// consecutive outputs per workgroup, RL_T terms of each per chunk, streamed
-// through an LDS ring of RL_D chunks by all RL_THREADS threads, RL_D - 1 chunks
-// ahead of wave 0, whose lane o adds output o's terms in order.
+// and every st1 bytes after it), with the loads spread over a workgroup: O
+// consecutive outputs per workgroup, T terms of each per chunk, streamed through an
+// LDS ring of D chunks by all RL_THREADS threads, D - 1 chunks ahead of wave 0, whose
+// lane o adds output o's terms in order. The first D - 1 chunks are asked for
+// together; each later one waits for its loads alone. So while few outputs leave
+// CUs idle, workgroups take 16 of them and long chunks (bound by the loads' latency:
+// 64 outputs and 32 terms -> 16 and 128: 4096 outputs of 512 terms 10.3 -> 6.8 us, 777
+// of 130 4.9 -> 3.9, 100 of 8192 128 -> 76); more outputs take 64, whole lines of
+// 256 bytes (16384 of 512 10.7 us, with 16 at a time 14.7).
 constexpr int RL_THREADS = 256;
-constexpr int RL_T = 32;
-constexpr int RL_D = 4;
-constexpr int RL_PER = RL_T * 64 / RL_THREADS;  // loads per thread and chunk
+constexpr int RL_MIN = 64;       // terms from which on
+constexpr int RL_AT_ONCE = 32;   // terms read from LDS ahead of their adds
+template <int RL_O, int RL_T, int RL_D>
 __global__ __launch_bounds__(RL_THREADS) void k_repeat_back_lds(const uint8_t* __restrict__ a, Shape4 sa,
                                                                 float* __restrict__ d, Shape4 sd) {
-    __shared__ float ring[RL_D * RL_T * 64];
+    constexpr int RL_STEP = RL_THREADS / RL_O;  // terms between two loads of a thread
+    constexpr int RL_PER = RL_T / RL_STEP;      // loads per thread and chunk
+    static_assert(RL_THREADS % RL_O == 0 && RL_O <= 64, "a thread loads one output's terms, wave 0 adds them");
+    static_assert(RL_T % RL_STEP == 0 && RL_T % RL_AT_ONCE == 0 && RL_D >= 3, "whole loads; one barrier per chunk");
+    __shared__ float ring[RL_D * RL_T * RL_O];
     const int64_t n = sd.ne[0] * sd.ne[1] * sd.ne[2] * sd.ne[3];
-    const int tid = threadIdx.x, o = tid % 64;
-    int64_t j = (int64_t) blockIdx.x * 64 + o;
+    const int tid = threadIdx.x, o = tid % RL_O;
+    int64_t j = (int64_t) blockIdx.x * RL_O + o;
     const bool valid = j < n;
     j = valid ? j : n - 1;  // outputs past the end re-read the last; nobody stores them
     const int64_t j0 = j % sd.ne[0], j1 = (j / sd.ne[0]) % sd.ne[1], j2 = (j / (sd.ne[0] * sd.ne[1])) % sd.ne[2],
@@ -720,43 +729,44 @@ __global__ __launch_bounds__(RL_THREADS) void k_repeat_back_lds(const uint8_t* _
     auto load = [&](int64_t c, float (&v)[RL_PER]) {
 #pragma unroll
         for (int u = 0; u < RL_PER; ++u) {
-            const int64_t q = c * RL_T + (tid + RL_THREADS * u) / 64;  // this load's term
+            const int64_t q = c * RL_T + tid / RL_O + RL_STEP * u;  // this load's term
             v[u] = *(const float*) (base + (q < terms ? q : terms - 1) * st1);
         }
     };
     auto store = [&](int64_t c, const float (&v)[RL_PER]) {
-        float* slot = ring + (int) (c % RL_D) * RL_T * 64;
+        float* slot = ring + (int) (c % RL_D) * RL_T * RL_O;
 #pragma unroll
         for (int u = 0; u < RL_PER; ++u) slot[tid + RL_THREADS * u] = v[u];  // [term][output]
     };
-    for (int64_t c = 0; c < RL_D - 1 && c < chunks; ++c) {
-        float v[RL_PER];
-        load(c, v);
-        store(c, v);
-    }
+    // (chunks past the last are its last term again, and nobody adds them)
+    float first[RL_D - 1][RL_PER];
+#pragma unroll
+    for (int c = 0; c < RL_D - 1; ++c) load(c, first[c]);
+#pragma unroll
+    for (int c = 0; c < RL_D - 1; ++c) store(c, first[c]);
     __syncthreads();
     float s = 0.f;
     for (int64_t c = 0; c < chunks; ++c) {
         float v[RL_PER];
         const bool more = c + RL_D - 1 < chunks;
         if (more) load(c + RL_D - 1, v);
-        if (tid < 64) {
-            const float* slot = ring + (int) (c % RL_D) * RL_T * 64;
-            const int64_t m = terms - c * RL_T < RL_T ? terms - c * RL_T : RL_T;
-            if (m == RL_T) {  // a whole chunk: every term read first, then added in order
-                float t[RL_T];
+        if (tid < RL_O) {
+            const float* slot = ring + (int) (c % RL_D) * RL_T * RL_O + o;
+            const int m = (int) (terms - c * RL_T < RL_T ? terms - c * RL_T : RL_T);
+            int q0 = 0;
+            for (; q0 + RL_AT_ONCE <= m; q0 += RL_AT_ONCE) {  // read together, then added in order
+                float t[RL_AT_ONCE];
 #pragma unroll
-                for (int q = 0; q < RL_T; ++q) t[q] = slot[q * 64 + o];
+                for (int q = 0; q < RL_AT_ONCE; ++q) t[q] = slot[(q0 + q) * RL_O];
 #pragma unroll
-                for (int q = 0; q < RL_T; ++q) s = s + t[q];
-            } else {
-                for (int64_t q = 0; q < m; ++q) s = s + slot[q * 64 + o];
+                for (int q = 0; q < RL_AT_ONCE; ++q) s = s + t[q];
             }
+            for (; q0 < m; ++q0) s = s + slot[q0 * RL_O];
         }
         __syncthreads();
         if (more) store(c + RL_D - 1, v);
     }
-    if (tid < 64 && valid) d[j] = s;
+    if (tid < RL_O && valid) d[j] = s;
 }
 
 // The same sums when ne0 is not repeated and each has few terms (the gradient of a
@@ -1113,9 +1123,16 @@ int launch_repeat_back_f32(const trc_hip_tensor& a, const trc_hip_tensor& d, hip
     if (!contiguous_f32(d)) return fail(TRC_HIP_E_SHAPE, "repeat_back: dst must be contiguous");
     if (!f32_aligned(a) || !f32_aligned(d)) return fail(TRC_HIP_E_ALIGN, "repeat_back: 4-byte alignment");
     const int64_t n = nelem(d);
-    if (a.ne[0] == d.ne[0] && a.ne[2] == d.ne[2] && a.ne[3] == d.ne[3] && a.ne[1] / d.ne[1] >= 2 * RL_T) {
-        hipLaunchKernelGGL(k_repeat_back_lds, dim3((unsigned) ((n + 63) / 64)), dim3(RL_THREADS), 0, s,
-                           (const uint8_t*) a.data, shape_of(a), (float*) d.data, shape_of(d));
+    if (a.ne[0] == d.ne[0] && a.ne[2] == d.ne[2] && a.ne[3] == d.ne[3] && a.ne[1] / d.ne[1] >= RL_MIN) {
+        // 16 outputs each while that is at most two workgroups a CU (10240 outputs of
+        // 128 terms 4.3 us either way)
+        if (n <= 32 * (int64_t) device_cus()) {
+            hipLaunchKernelGGL((k_repeat_back_lds<16, 128, 3>), dim3((unsigned) ((n + 15) / 16)), dim3(RL_THREADS), 0, s,
+                               (const uint8_t*) a.data, shape_of(a), (float*) d.data, shape_of(d));
+        } else {
+            hipLaunchKernelGGL((k_repeat_back_lds<64, 32, 4>), dim3((unsigned) ((n + 63) / 64)), dim3(RL_THREADS), 0, s,
+                               (const uint8_t*) a.data, shape_of(a), (float*) d.data, shape_of(d));
+        }
         return check_launch("repeat_back");
     }
     const int64_t r1 = a.ne[1] / d.ne[1], r2 = a.ne[2] / d.ne[2], r3 = a.ne[3] / d.ne[3];
