@@ -45,7 +45,9 @@ ROOT = Path(__file__).resolve().parent
 PKG = ROOT / "train.cpp_amd"
 
 HBM_PEAK_GBS = 8000.0        # MI355X HBM3E, GB/s
-FP32_MFMA_PEAK_TFS = 157.3   # MI355X dense FP32 matrix, TFLOP/s
+# MI355X dense FP32 matrix, TFLOP/s. F32 products run on the bf16 matrix cores, each
+# float as three bf16, so their share of this rate can exceed 1.
+FP32_MFMA_PEAK_TFS = 157.3
 METRIC = "Q4_0 dequant-matvec GB/s (% HBM peak); F32 mul_mat TFLOP/s (% MFMA peak)"
 
 
