@@ -80,6 +80,22 @@ def test_cpy_transpose_tiles(hip, shape):
     out.free()
 
 
+@pytest.mark.parametrize("ne0", [2, 63, 64, 65])
+@pytest.mark.parametrize("ne1", [2, 63, 65, 333])
+def test_cpy_transpose_tile_edges(hip, ne0, ne1):
+    """Tiles cut at either edge, down to two rows, with the planes of src permuted."""
+    announce(f"abi cpy transpose edges {ne0} x {ne1}")
+    x = np.random.default_rng(32).standard_normal((2, 3, ne0, ne1)).astype(np.float32)
+    src = Dev(x)
+    view = src.base.transpose(1, 0, 3, 2)
+    out = empty(view.shape, np.float32)
+    H.cpy(src.tensor(view), out.tensor())
+    H.sync()
+    assert np.array_equal(out.read().view(np.uint32), np.ascontiguousarray(x.transpose(1, 0, 3, 2)).view(np.uint32))
+    src.free()
+    out.free()
+
+
 def test_forced_error_hook(hip):
     os.environ["TRC_HIP_FORCE_ERROR"] = "trc_hip_dequant"
     try:

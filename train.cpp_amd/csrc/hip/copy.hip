@@ -79,7 +79,11 @@ __global__ __launch_bounds__(CP_THREADS) void k_cpy(const uint8_t* __restrict__ 
 // The same copy for 4-byte elements when src runs along dim 1 (nb1 == 4, the
 // transposed views autograd builds) and dst along dim 0 (nb0 == 4): 64 x 64
 // tiles of (i0, i1) go through LDS, read as 256-byte runs of src along i1 and
-// written as 256-byte runs of dst along i0.
+// written as 256-byte runs of dst along i0. Bound by the loads' latency where tiles
+// are few: a thread asks for its 16 elements together, from addresses clamped into
+// the tensor (each behind a branch of its own, they waited one for another:
+// [64, 333, 12, 2] 4.7 -> 3.3 us with its operands in cache, 10 -> 4 without; 4095 x
+// 4097 27.8 -> 23.9).
 constexpr int TT = 64;
 __global__ __launch_bounds__(CP_THREADS) void k_cpy_transpose(const uint8_t* __restrict__ src,
                                                              uint8_t* __restrict__ dst, int64_t ne0, int64_t ne1,
@@ -97,11 +101,16 @@ __global__ __launch_bounds__(CP_THREADS) void k_cpy_transpose(const uint8_t* __r
     uint8_t* dp = dst + i2 * dnb2 + i3 * dnb3;
     const int64_t b0 = t0 * TT, b1 = t1 * TT;
     const int lane = threadIdx.x % TT, row = threadIdx.x / TT;  // 4 rows per pass
+    constexpr int STEP = CP_THREADS / TT;
+    uint32_t v[TT / STEP];
+    sp += (b1 + lane < ne1 ? b1 + lane : ne1 - 1) * 4;
 #pragma unroll
-    for (int k = 0; k < TT; k += CP_THREADS / TT) {
-        const int64_t i0 = b0 + row + k, i1 = b1 + lane;
-        if (i0 < ne0 && i1 < ne1) tile[row + k][lane] = *(const uint32_t*) (sp + i0 * snb0 + i1 * 4);
+    for (int k = 0; k < TT / STEP; ++k) {
+        const int64_t i0 = b0 + row + k * STEP;
+        v[k] = *(const uint32_t*) (sp + (i0 < ne0 ? i0 : ne0 - 1) * snb0);
     }
+#pragma unroll
+    for (int k = 0; k < TT / STEP; ++k) tile[row + k * STEP][lane] = v[k];
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < TT; k += CP_THREADS / TT) {
