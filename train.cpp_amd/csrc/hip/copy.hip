@@ -82,8 +82,8 @@ __global__ __launch_bounds__(CP_THREADS) void k_cpy(const uint8_t* __restrict__ 
 // written as 256-byte runs of dst along i0. Bound by the loads' latency where tiles
 // are few: a thread asks for its 16 elements together, from addresses clamped into
 // the tensor (each behind a branch of its own, they waited one for another:
-// [64, 333, 12, 2] 4.7 -> 3.3 us with its operands in cache, 10 -> 4 without; 4095 x
-// 4097 27.8 -> 23.9).
+// [64, 333, 12, 2] 4.7 -> 3.3 us again and again on one tensor, 6 us less of a pass
+// whose product has just written it; 4095 x 4097 27.8 -> 23.9).
 constexpr int TT = 64;
 __global__ __launch_bounds__(CP_THREADS) void k_cpy_transpose(const uint8_t* __restrict__ src,
                                                              uint8_t* __restrict__ dst, int64_t ne0, int64_t ne1,
