@@ -613,3 +613,53 @@ def test_bf16_tiles_without_a_workspace(hip):
     for a, b, d in cases:
         for x in (a, b, d):
             x.free()
+
+
+# ---------------------------------------------------------------- strides of tens of megabytes
+
+@pytest.mark.parametrize("acc", [False, True], ids=["plain", "acc"])
+@pytest.mark.parametrize("shape", [(1024, 4096, 5), (1024, 2000, 2)])
+def test_dst_columns_far_apart(hip, shape, acc):
+    """Few dst columns 100 MB and more apart: the kernels form offsets for up to 28
+    columns, and those of columns that are not there pass 2^31 and 2^32. Nothing but
+    the columns is written, and they hold the product."""
+    K, M, N = shape
+    stride = 400_000_000 // (N - 1)                    # bytes; 27 of them pass 2^31 (N = 2: 2^32 too)
+    announce(f"mul_mat dst columns {stride} bytes apart {shape} {'acc' if acc else ''}")
+    A = synth.normal(980 + N, K * M).reshape(1, 1, K, M)   # row-contiguous: tiles, not the few-column kernel
+    B = synth.normal(981 + N, K * N).reshape(1, 1, N, K)
+    da, db = Dev(A), Dev(B)
+    total = stride // 4 * (N - 1) + M
+    buf = H.DeviceBuffer(4 * total)
+    H.fill_f32(buf.ptr, 0.5, total)
+    d = H.tensor(buf.ptr, [M, N, 1, 1], [4, stride, stride * N, stride * N])
+    (H.mul_mat_acc_f32 if acc else H.mul_mat_f32)(da.tensor(t01(A)), db.tensor(), d)
+    H.sync()
+    out = buf.download(np.empty(total, np.float32))
+    for x in (da, db, buf):
+        x.free()
+    cols = [out[j * (stride // 4):j * (stride // 4) + M] for j in range(N)]
+    got = np.stack(cols)[None, None]
+    want = O.mul_mat(t01(A), B, threads=8)
+    assert O.row_l2_error(got, want + np.float32(0.5) if acc else want) <= TOL
+    for c in cols:
+        c[:] = 0.5
+    assert np.all(out == np.float32(0.5))
+
+
+def test_operand_rows_far_apart(hip):
+    """A transposed operand with 80 MB from one k to the next: the loads form offsets
+    up to the end of the last slab of 32 k, past 2^31."""
+    K, M, N, stride = 20, 4096, 4096, 80_000_000
+    announce("mul_mat src0 with k 80 MB apart")
+    A, B = synth.normal(985, K * M).reshape(K, M), synth.normal(986, K * N).reshape(1, 1, N, K)
+    buf = H.DeviceBuffer(stride * (K - 1) + 4 * M)
+    for k in range(K):
+        H.check(H.load().trc_hip_h2d(buf.ptr + k * stride, A[k].ctypes.data, 4 * M, None))
+    db, out = Dev(B), empty((1, 1, N, M))
+    H.mul_mat_f32(H.tensor(buf.ptr, [K, M, 1, 1], [stride, 4, 4 * M, 4 * M]), db.tensor(), out.tensor())
+    H.sync()
+    got = out.read()
+    for x in (buf, db, out):
+        x.free()
+    assert O.row_l2_error(got, O.mul_mat(t01(A[None, None]), B, threads=8)) <= TOL

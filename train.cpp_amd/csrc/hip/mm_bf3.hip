@@ -8,11 +8,14 @@ int launch_mm_bf3_pair(const MMArgs& p, unsigned grid, hipStream_t s);
 int launch_mm_bf3_slots(const MMArgs& p, unsigned grid, hipStream_t s);
 
 bool mm_bf3_fits(const MMArgs& p) {
-    // 32-bit buffer offsets over the rows of a tile
+    // 32-bit buffer offsets over the rows of a tile, those included that are formed
+    // for what is not there: k up to the end of its slab, and the columns of a wave's
+    // 32 x 32 block, the last 27 after the one its lanes' offsets name
     auto span = [](int64_t n0, int64_t nb0, int64_t n1, int64_t nb1) { return (n0 - 1) * nb0 + (n1 - 1) * nb1 + 4; };
+    const int64_t k = (p.K + 31) / 32 * 32;
     const int64_t ti = p.M < B3_T ? p.M : B3_T, tj = p.N < B3_T ? p.N : B3_T;
-    return span(p.K, p.a_nb0, ti, p.a_nb1) <= MM_PAST && span(p.K, p.b_nb0, tj, p.b_nb1) <= MM_PAST &&
-           span(ti, p.d_nb0, tj, p.d_nb1) <= MM_PAST;
+    return span(k, p.a_nb0, ti, p.a_nb1) <= MM_PAST && span(k, p.b_nb0, tj, p.b_nb1) <= MM_PAST &&
+           span(ti, p.d_nb0, tj < 28 ? 28 : tj, p.d_nb1) <= MM_PAST;
 }
 
 B3Plan mm_bf3_plan(const MMArgs& p, int64_t planes, int max_parts) {

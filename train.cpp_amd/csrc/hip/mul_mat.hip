@@ -241,6 +241,8 @@ __global__ __launch_bounds__(WI * WJ * 64) void k_mul_mat(MMArgs p) {
         // plus uniform multiples of nb1, and rows or columns past dst get an
         // offset past the resource (reads 0, stores dropped), so there is no
         // branch and each block's accumulators are read only when it is stored.
+        // (A column that is not there adds no multiple of nb1: 27 of them can
+        // pass 4 GiB, and the sum would be an offset into dst again.)
         const __amdgpu_buffer_rsrc_t rd =
             __builtin_amdgcn_make_buffer_rsrc((void*) d, (short) 0, (int) p.d_span, MM_RSRC_WORD3);
 #pragma unroll
@@ -266,19 +268,17 @@ __global__ __launch_bounds__(WI * WJ * 64) void k_mul_mat(MMArgs p) {
                 } else {  // the tile's last columns lie past dst: four at a time (fewer offsets held)
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-#pragma unroll
-                        for (int v = 4 * q; v < 4 * q + 4; ++v) {
+                        auto off = [&](int v) {
                             const int c = 8 * (v >> 2) + (v & 3);
-                            old[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                                   rd, jb + c < p.N ? vo : MM_OUT, (uint32_t) (c * p.d_nb1), 0));
-                        }
+                            return vo != MM_OUT && jb + c < p.N ? vo + (uint32_t) (c * p.d_nb1) : MM_OUT;
+                        };
 #pragma unroll
-                        for (int v = 4 * q; v < 4 * q + 4; ++v) {
-                            const int c = 8 * (v >> 2) + (v & 3);
+                        for (int v = 4 * q; v < 4 * q + 4; ++v)
+                            old[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, off(v), 0, 0));
+#pragma unroll
+                        for (int v = 4 * q; v < 4 * q + 4; ++v)
                             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, old[v] + acc[x][y][v]),
-                                                                  rd, jb + c < p.N ? vo : MM_OUT,
-                                                                  (uint32_t) (c * p.d_nb1), 0);
-                        }
+                                                                  rd, off(v), 0, 0);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
