@@ -65,6 +65,7 @@ def runtime() -> C.CDLL:
             "hipStreamCreate": [PV], "hipStreamDestroy": [V], "hipStreamBeginCapture": [V, C.c_int],
             "hipStreamEndCapture": [V, PV], "hipGraphInstantiate": [PV, V, V, V, C.c_size_t],
             "hipGraphLaunch": [V, V], "hipGraphExecDestroy": [V], "hipGraphDestroy": [V],
+            "hipGraphGetNodes": [V, PV, C.POINTER(C.c_size_t)], "hipGraphKernelNodeGetParams": [V, V],
             "hipMemGetInfo": [C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)], "hipDeviceSynchronize": [],
             "hipGetLastError": [],
         }.items():
@@ -101,3 +102,37 @@ class Stream:
             H.sync(self.handle)
             assert runtime().hipStreamDestroy(C.c_void_p(self.handle)) == 0
             self.handle = None
+
+
+class _KernelNode(C.Structure):  # hipKernelNodeParams
+    _fields_ = [("block", C.c_uint32 * 3), ("extra", C.c_void_p), ("func", C.c_void_p), ("grid", C.c_uint32 * 3),
+                ("params", C.c_void_p), ("shared", C.c_uint32)]
+
+
+def launches(fn) -> list[tuple[int, int]]:
+    """(workgroups, threads of one) of every kernel that fn(stream) launches, read
+    from a capture of it; fn runs once before, so that the stream has its workspaces."""
+    rt = runtime()
+    s = Stream()
+    try:
+        fn(s.handle)
+        H.sync(s.handle)
+        graph = C.c_void_p()
+        assert rt.hipStreamBeginCapture(C.c_void_p(s.handle), 0) == 0
+        try:
+            fn(s.handle)
+        finally:
+            rc = rt.hipStreamEndCapture(C.c_void_p(s.handle), C.byref(graph))
+        assert rc == 0
+        n = C.c_size_t(64)
+        nodes = (C.c_void_p * 64)()
+        assert rt.hipGraphGetNodes(graph, nodes, C.byref(n)) == 0
+        out = []
+        for i in range(n.value):
+            k = _KernelNode()
+            assert rt.hipGraphKernelNodeGetParams(C.c_void_p(nodes[i]), C.byref(k)) == 0
+            out.append((k.grid[0] * k.grid[1] * k.grid[2], k.block[0] * k.block[1] * k.block[2]))
+        assert rt.hipGraphDestroy(graph) == 0
+        return out
+    finally:
+        s.close()

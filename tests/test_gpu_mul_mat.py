@@ -10,7 +10,7 @@ import pytest
 
 import oracle_lib as O
 from conftest import GOLDEN, announce
-from gpu_util import Dev, Stream, empty, gpu_mul_mat
+from gpu_util import Dev, Stream, empty, gpu_mul_mat, launches
 from traincpp_amd import hip as H
 from traincpp_amd import synth
 
@@ -613,6 +613,51 @@ def test_bf16_tiles_without_a_workspace(hip):
     for a, b, d in cases:
         for x in (a, b, d):
             x.free()
+
+
+def bf16_route(a, b, d, acc=False):
+    """How a product on 256-CU devices is launched: "whole8" or "whole4" (bf16 tiles, K
+    whole, workgroups of 8 or 4 waves), "pair" (K in two parts that meet in dst), "slots"
+    (more parts), or "fp32" (another grid). From 512 tiles of 128 x 128 on the FP32
+    tiles' grid is that of "whole4": shapes here have fewer."""
+    f = H.mul_mat_acc_f32 if acc else H.mul_mat_f32
+    (grid, block), = launches(lambda s: f(a, b, d, s))
+    tiles = -(-d.ne[0] // 128) * -(-d.ne[1] // 128) * d.ne[2] * d.ne[3]
+    if grid % tiles or (block == 256) != (grid == tiles and tiles > 256):
+        return "fp32"
+    return {1: "whole4" if block == 256 else "whole8", 2: "pair"}.get(grid // tiles, "slots")
+
+
+@pytest.mark.parametrize("which", ["src0", "src1"])
+@pytest.mark.parametrize("shape", [
+    # (K, M, N, accumulated, route): rows of 1, 2 and 3 past a multiple of four
+    (1056, 1409, 1410, False, "whole8"), (200, 2689, 2690, False, "whole4"), (1000, 1409, 1411, True, "whole8"),
+    (1056, 1281, 1283, False, "pair"), (1056, 777, 130, False, "slots"),
+])
+def test_transposed_operands_ignore_what_follows_their_rows(hip, shape, which):
+    """A transposed view of a wider buffer whose row count is no multiple of four: the
+    loads of four rows reach into the columns after the view. Nothing there may matter,
+    NaN, infinity or subnormal: the bits are those with zeros there."""
+    K, M, N, acc, route = shape
+    announce(f"mul_mat transposed view with padding {shape} {which}")
+    rng = np.random.default_rng(K + M)
+    A, B = (rng.standard_normal((1, 1, K, r + 3)).astype(np.float32) for r in (M, N))
+    out, bits = empty((1, 1, N, M)), []
+    for pad in (0.0, np.nan, np.inf, 1e-40):
+        (A if which == "src0" else B)[..., -3:] = pad
+        da, db = Dev(A), Dev(B)
+        ta, tb = da.tensor(t01(A[..., :M])), db.tensor(t01(B[..., :N]))
+        H.fill_f32(out.ptr, 0.0, M * N)
+        (H.mul_mat_acc_f32 if acc else H.mul_mat_f32)(ta, tb, out.tensor())
+        H.sync()
+        bits.append(out.read().view(np.uint32))
+        if pad == 0.0:
+            assert bf16_route(ta, tb, out.tensor(), acc) == route
+            assert _rel(bits[0].view(np.float32), _f64(t01(A[..., :M]), t01(B[..., :N]))) <= 2.0 ** -25 * np.sqrt(K)
+        da.free()
+        db.free()
+    out.free()
+    assert all(np.array_equal(bits[0], x) for x in bits[1:])
 
 
 # ---------------------------------------------------------------- strides of tens of megabytes
