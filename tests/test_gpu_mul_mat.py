@@ -660,6 +660,69 @@ def test_transposed_operands_ignore_what_follows_their_rows(hip, shape, which):
     assert all(np.array_equal(bits[0], x) for x in bits[1:])
 
 
+def laid(x, layout):
+    """(a buffer, the view of it that is x) with x's rows along k ("k"), its columns
+    ("t": a transposed view), rows along k off 16-byte alignment ("odd"), or neither
+    ("gen": every other element along both)."""
+    if layout == "t":
+        base = np.ascontiguousarray(t01(x))
+        return base, t01(base)
+    if layout == "odd":
+        base = np.zeros(x.shape[:3] + (x.shape[3] + 3,), np.float32)
+        view = base[..., 3:]
+    elif layout == "gen":
+        base = np.zeros(x.shape[:2] + (2 * x.shape[2], 2 * x.shape[3]), np.float32)
+        view = base[:, :, ::2, ::2]
+    else:
+        return x, x
+    view[:] = x
+    return base, view
+
+
+def bf16_run(A, B, layouts, acc, route):
+    """The product (added into zeros where acc) of A and B laid out as given, whose
+    launch is asserted to be `route`."""
+    (ab, av), (bb, bv) = laid(A, layouts[0]), laid(B, layouts[1])
+    da, db, out = Dev(ab), Dev(bb), empty((1, B.shape[1], B.shape[2], A.shape[2]))
+    ta, tb, td = da.tensor(av), db.tensor(bv), out.tensor()
+    assert bf16_route(ta, tb, td, acc) == route
+    H.fill_f32(out.ptr, 0.0, out.base.size)
+    (H.mul_mat_acc_f32 if acc else H.mul_mat_f32)(ta, tb, td)
+    H.sync()
+    got = out.read()
+    for d in (da, db, out):
+        d.free()
+    return got
+
+
+# (K, M, N, accumulated, route): one shape for each way the parts of K come together
+BF16_ONE_EACH = [(1056, 1409, 1410, False, "whole8"), (200, 2689, 2690, False, "whole4"), (1000, 1409, 1411, True, "whole8"),
+                 (200, 2691, 2689, True, "whole4"), (1056, 1281, 1283, False, "pair"), (1056, 777, 130, False, "slots")]
+
+
+@pytest.mark.parametrize("layouts", ["kk", "tt"])
+@pytest.mark.parametrize("shape", BF16_ONE_EACH)
+def test_bf16_tiles_small_values(hip, shape, layouts):
+    """Operands down to the smallest float take the same way as any other: scaled by
+    powers of two, normal floats near 2^-115 give the scaled result's bits, and
+    integer multiples of powers of two whose sums a float holds give exact sums where
+    the operand, its products or the results are subnormal."""
+    K, M, N, acc, route = shape
+    announce(f"mul_mat bf16 tiles small values {shape} {layouts}")
+    rng = np.random.default_rng(K + N)
+    A, B = ((1 + rng.random((1, 1, r, K))).astype(np.float32) * rng.choice([-1, 1], (1, 1, r, K)).astype(np.float32)
+            for r in (M, N))
+    run = lambda a, b: bf16_run(a.astype(np.float32), b.astype(np.float32), layouts, acc, route)
+    plain = run(A, B)
+    assert np.array_equal(run(A * 2.0 ** -115, B * 2.0 ** 60).view(np.uint32), np.ldexp(plain, -55).view(np.uint32))
+    assert np.array_equal(run(A * 2.0 ** 30, B * 2.0 ** -120).view(np.uint32), np.ldexp(plain, -90).view(np.uint32))
+    A, B = (rng.integers(-40, 41, (1, 1, r, K)).astype(np.float64) for r in (M, N))
+    want = _f64(A, B)
+    assert np.abs(want).max() < 2 ** 22
+    for ea, eb in [(-149, 40), (20, -149), (-70, -79), (-140, 5)]:  # the last two: results of 2^-149 and 2^-135 up
+        assert np.array_equal(run(A * 2.0 ** ea, B * 2.0 ** eb), (want * 2.0 ** (ea + eb)).astype(np.float32))
+
+
 # ---------------------------------------------------------------- strides of tens of megabytes
 
 @pytest.mark.parametrize("acc", [False, True], ids=["plain", "acc"])

@@ -15,11 +15,17 @@
 // 1.15e-6 -> 0.40e-6 (positive inputs at K = 4096 1.01e-6 -> 0.35e-6), and the
 // mean error is as near 0 (K = 4096: 2e-8 -> 5e-9 of the result's 2-norm).
 //
-// What the split cannot hold is computed again: l is exact unless its low 16
-// float bits are set (|x| under about 2^-110) or x is not finite or rounds to
-// infinity as bf16, which leaves a result that is not finite. A workgroup that
-// finds either repeats its tile with the FP32 instructions, so infinities, NaNs,
-// overflows and values near the smallest float come out as those give them.
+// Operands are split as x 2^24 and results scaled back by 2^-48, both exact: every
+// part is then 0 or at least 2^-125, a normal bf16, down to the smallest
+// subnormal float, so that small values (the tails of a softmax) are held like any
+// other. What the split cannot hold is at the other end: x not finite or 2^104 and
+// more, or sums from 2^80 on, which leave a result that is not finite. A workgroup
+// that finds one repeats its tile with the FP32 instructions, so infinities, NaNs
+// and overflows come out as those give them, at the price of both passes: 4096 x
+// 4096 x 512 with one infinity 229 us, without 92 (FP32 instructions alone 140).
+// (Unscaled, the same repeat was needed for any value under about 2^-110: the
+// product with softmax weights of that shape took 238 us, now 92. Nothing that
+// would have to be gathered in the loop stays either, and no register spills.)
 #pragma once
 
 #include "common.h"
@@ -51,15 +57,16 @@ __device__ __forceinline__ uint32_t b3_cvt(float a, float b) {
 __device__ __forceinline__ float b3_lo(uint32_t p) { return __builtin_bit_cast(float, p << 16); }
 __device__ __forceinline__ float b3_hi(uint32_t p) { return __builtin_bit_cast(float, p & 0xFFFF0000u); }
 
-// Two floats (consecutive k of one row) as three packed bf16 pairs; `lost`
-// gathers the bits of the last parts that bf16 cannot hold (low 16).
-__device__ __forceinline__ void b3_split(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l, uint32_t& lost) {
+// Two floats (consecutive k of one row) times 2^24 as three packed bf16 pairs.
+constexpr float B3_UP = 0x1p24f, B3_DOWN = 0x1p-48f;
+__device__ __forceinline__ void b3_split(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
+    x *= B3_UP;
+    y *= B3_UP;
     h = b3_cvt(x, y);
     const float rx = x - b3_lo(h), ry = y - b3_hi(h);
     m = b3_cvt(rx, ry);
     const uint32_t sx = __builtin_bit_cast(uint32_t, rx - b3_lo(m)), sy = __builtin_bit_cast(uint32_t, ry - b3_hi(m));
     l = __builtin_amdgcn_perm(sy, sx, 0x07060302u);
-    lost |= sx | sy;
 }
 
 // One operand's slab: 128 rows x 16 G k, 8 floats per thread (256 G threads).
@@ -167,12 +174,12 @@ struct B3Slab {
     }
     // half u of the registers, split, into the planes at l: piece u, or
     // (R_CONTIG) rows 2u and 2u + 1 of the four, whose k pair is in both pieces
-    __device__ __forceinline__ void store(int st, uint8_t* l, int u, uint32_t& lost) const {
+    __device__ __forceinline__ void store(int st, uint8_t* l, int u) const {
         if constexpr (MODE == MM_R_CONTIG) {
 #pragma unroll
             for (int j = 2 * u; j < 2 * u + 2; ++j) {
                 uint32_t h, m, t;
-                b3_split(r[st][0][j], r[st][1][j], h, m, t, lost);
+                b3_split(r[st][0][j], r[st][1][j], h, m, t);
                 uint8_t* d = l + lo + j * RS;
                 *(uint32_t*) d = h;
                 *(uint32_t*) (d + PS) = m;
@@ -181,9 +188,9 @@ struct B3Slab {
         } else {
             u2 h, m, t;
             uint32_t a, b, c;
-            b3_split(r[st][u].x, r[st][u].y, a, b, c, lost);
+            b3_split(r[st][u].x, r[st][u].y, a, b, c);
             h.x = a, m.x = b, t.x = c;
-            b3_split(r[st][u].z, r[st][u].w, a, b, c, lost);
+            b3_split(r[st][u].z, r[st][u].w, a, b, c);
             h.y = a, m.y = b, t.y = c;
             uint8_t* d = l + lo + u * 64 * 16;
             *(u2*) d = h;
@@ -280,7 +287,6 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[x][y][v] = 0.f;
     };
-    uint32_t lost = 0;
     auto gload = [&](int st, int kt) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
@@ -291,8 +297,8 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
     auto lstore = [&](int st, uint8_t* l) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            sa.store(st, l, u, lost);
-            sb.store(st, l + SA::BYTES, u, lost);
+            sa.store(st, l, u);
+            sb.store(st, l + SA::BYTES, u);
         }
     };
     auto mask_rows = [&](int st) {
@@ -377,10 +383,10 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
                     f16v& c = q < 5 ? cor[x][y] : acc[x][y];
                     c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[PB[q]][y], fa[PA[q]][x], c, 0, 0, 0);
                 }
-            if (q == 1) fragsA(rd, 2), sa.store(ST, nxt, 0, lost);
-            if (q == 2) fragsB(rd, 2), sa.store(ST, nxt, 1, lost);
-            if (q == 3) fragsA(rd, 1), sb.store(ST, nxt + SA::BYTES, 0, lost);
-            if (q == 4) fragsB(rd, 1), sb.store(ST, nxt + SA::BYTES, 1, lost);
+            if (q == 1) fragsA(rd, 2), sa.store(ST, nxt, 0);
+            if (q == 2) fragsB(rd, 2), sa.store(ST, nxt, 1);
+            if (q == 3) fragsA(rd, 1), sb.store(ST, nxt + SA::BYTES, 0);
+            if (q == 4) fragsB(rd, 1), sb.store(ST, nxt + SA::BYTES, 1);
             if (q == 5) fragsA(rd, 0), fragsB(rd, 0);
             if constexpr (!decltype(last)::value) {
                 if (q == 2) sa.load(ST, kt + 4, nk, 0), sa.load(ST, kt + 4, nk, 1);
@@ -416,8 +422,7 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
         slab(kt + 1, one{}, std::true_type{});
     }
 
-    // what three bf16 could not hold, or a result that is not finite: the same
-    // sums on the FP32 instructions
+    // a result that is not finite: the same sums on the FP32 instructions
     float most = 0.f;  // of the results' magnitudes, NaN where one is
 #pragma unroll
     for (int x = 0; x < 2; ++x)
@@ -425,10 +430,10 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
         for (int y = 0; y < NY; ++y)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                acc[x][y][v] += cor[x][y][v];
+                acc[x][y][v] = (acc[x][y][v] + cor[x][y][v]) * B3_DOWN;
                 most = __builtin_elementwise_maximum(most, __builtin_fabsf(acc[x][y][v]));
             }
-    if (__syncthreads_or((lost & 0xFFFFu) != 0 || !(most < __builtin_inff()))) {
+    if (__syncthreads_or(!(most < __builtin_inff()))) {
         clear();
         float* la = (float*) lds;
         float* lb = la + BK * SA::LDF;
