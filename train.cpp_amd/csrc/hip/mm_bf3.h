@@ -82,11 +82,10 @@ __device__ __forceinline__ void b3_split(float x, float y, uint32_t& h, uint32_t
 //    consecutive rows fall on different banks.
 //  - GENERIC: K_CONTIG's mapping, element by element.
 // Loads go through a buffer resource over the plane: rows past the operand get
-// an offset past it (read 0), k past K is set to 0 where the last slab is
-// converted, and so are the rows past the operand of an R_CONTIG quad that holds
-// its last row too (what lies there belongs to others, and a NaN or an infinity
-// there must not send the tile to the FP32 instructions). 4-byte alignment is
-// enough for the 16-byte loads.
+// an offset past it (read 0), and k past K is set to 0 where the last slab is
+// converted. An R_CONTIG quad that holds the operand's last row may hold up to
+// three rows after it, whatever lies there: they reach only sums outside dst.
+// 4-byte alignment is enough for the 16-byte loads.
 template <int MODE, int G>
 struct B3Slab {
     static constexpr int RS = MODE == MM_R_CONTIG ? 32 * 16 + 32 : 0;
@@ -98,8 +97,6 @@ struct B3Slab {
     uint32_t lo;     // LDS byte offset of piece 0
     uint32_t nb0;
     uint32_t step;   // bytes from one slab to the next
-    bool cut;        // R_CONTIG: the tile's rows are no multiple of 4 (uniform)
-    int have;        // R_CONTIG: rows from the thread's first on
     __amdgpu_buffer_rsrc_t rs;
     f4 r[2][2];      // [stage][piece]: slab s waits in stage s % 2
 
@@ -116,7 +113,6 @@ struct B3Slab {
                                                (int) ((rows - 1) * nbr + (K - 1) * nbk + 4), MM_RSRC_WORD3);
         nb0 = (uint32_t) nbk;
         step = (uint32_t) (16 * G * nbk);
-        cut = MODE == MM_R_CONTIG && (rows & 3) != 0;
         if constexpr (MODE == MM_R_CONTIG) {
             const int lane = tid & 63, wave = tid >> 6;
             const int q = 8 * (wave & 3) + (lane & 7), kp = (lane >> 3) & 7, g = wave >> 2;
@@ -126,7 +122,6 @@ struct B3Slab {
                 vo[u] = 4 * q < rows ? (uint32_t) ((k0 + ko[u]) * nbk + 16 * q) : MM_OUT;
             }
             lo = (uint32_t) (g * GS + (kp >> 2) * HS + q * 16 + (kp & 3) * 4);
-            have = rows - 4 * q;
         } else {
             const int row = tid / (4 * G), kq = tid % (4 * G);
 #pragma unroll
@@ -159,18 +154,6 @@ struct B3Slab {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (ko[u] + (MODE == MM_R_CONTIG ? 0 : e) >= left) r[st][u][e] = 0.f;
-    }
-    // the rows past the operand become 0
-    __device__ __forceinline__ void mask_rows(int st) {
-        if constexpr (MODE == MM_R_CONTIG) {
-            if (cut) {
-#pragma unroll
-                for (int u = 0; u < 2; ++u)
-#pragma unroll
-                    for (int e = 1; e < 4; ++e)
-                        if (e >= have) r[st][u][e] = 0.f;
-            }
-        }
     }
     // half u of the registers, split, into the planes at l: piece u, or
     // (R_CONTIG) rows 2u and 2u + 1 of the four, whose k pair is in both pieces
@@ -301,10 +284,6 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
             sb.store(st, l + SA::BYTES, u);
         }
     };
-    auto mask_rows = [&](int st) {
-        sa.mask_rows(st);
-        sb.mask_rows(st);
-    };
     auto masked = [&](int st, int kt) {
         if (kt == nk - 1 && left < BK) {
             sa.mask(st, left);
@@ -326,7 +305,6 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
         masked(st, st);
-        mask_rows(st);
         lstore(st, lds + st * BUF);
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
@@ -371,7 +349,6 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
         const uint8_t* rd = lds + b1;
         uint8_t* nxt = lds + b2;
         if constexpr (decltype(last)::value) masked(ST, kt + 2);
-        mask_rows(ST);
         // m m, l h, h l, m h, h m into the small sums, h h into the large ones
         constexpr int PA[6] = {1, 2, 0, 1, 0, 0}, PB[6] = {1, 0, 2, 0, 1, 0};
 #pragma unroll
@@ -422,17 +399,28 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
         slab(kt + 1, one{}, std::true_type{});
     }
 
-    // a result that is not finite: the same sums on the FP32 instructions
+    // accumulator register v of tile (x, y) holds the tile's dst row i = ib + 32 x +
+    // col and column j = jb + 64 y + 8 (v / 4) + 4 half + v % 4
+    const int ib = wi * 64, jb = wj * 32;
+    const int rows = p.M - i0 < B3_T ? (int) (p.M - i0) : B3_T, cols = p.N - j0 < B3_T ? (int) (p.N - j0) : B3_T;
+    // a result that is not finite: the same sums on the FP32 instructions. Sums
+    // outside dst don't count (they can hold rows that are not the operand's).
     float most = 0.f;  // of the results' magnitudes, NaN where one is
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int x = 0; x < 2; ++x) {
+        float mx = 0.f;
 #pragma unroll
-        for (int y = 0; y < NY; ++y)
+        for (int y = 0; y < NY; ++y) {
+            const int rest = cols - (jb + y * 64 + 4 * half);
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 acc[x][y][v] = (acc[x][y][v] + cor[x][y][v]) * B3_DOWN;
-                most = __builtin_elementwise_maximum(most, __builtin_fabsf(acc[x][y][v]));
+                if (cols == B3_T || 8 * (v >> 2) + (v & 3) < rest)
+                    mx = __builtin_elementwise_maximum(mx, __builtin_fabsf(acc[x][y][v]));
             }
+        }
+        if (ib + x * 32 + col < rows) most = __builtin_elementwise_maximum(most, mx);
+    }
     if (__syncthreads_or(!(most < __builtin_inff()))) {
         clear();
         float* la = (float*) lds;
@@ -440,7 +428,6 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
         for (int k0 = 0; k0 < nk; ++k0) {
             gload(0, k0);
             masked(0, k0);
-            mask_rows(0);
             sa.store_f32(la, tid);
             sb.store_f32(lb, tid);
             __syncthreads();
@@ -459,9 +446,6 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
         }
     }
 
-    // accumulator register v of tile (x, y) holds the tile's dst row i = ib + 32 x +
-    // col and column j = jb + 64 y + 8 (v / 4) + 4 half + v % 4
-    const int ib = wi * 64, jb = wj * 32;
     constexpr int NX = G == 2 ? 1 : 2;
     int x0 = 0;
     if constexpr (G == 2) {
@@ -494,7 +478,6 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
                 for (int v = 0; v < 16; ++v) acc[0][y][v] = red[(32 + y * 16 + v) * 64] + acc[1][y][v];
         }
     }
-    const int rows = p.M - i0 < B3_T ? (int) (p.M - i0) : B3_T, cols = p.N - j0 < B3_T ? (int) (p.N - j0) : B3_T;
     d += i0 * p.d_nb0 + j0 * p.d_nb1;
     const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(
         (void*) d, (short) 0, (int) ((rows - 1) * p.d_nb0 + (cols - 1) * p.d_nb1 + 4), MM_RSRC_WORD3);
