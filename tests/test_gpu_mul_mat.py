@@ -723,6 +723,25 @@ def test_bf16_tiles_small_values(hip, shape, layouts):
         assert np.array_equal(run(A * 2.0 ** ea, B * 2.0 ** eb), (want * 2.0 ** (ea + eb)).astype(np.float32))
 
 
+@pytest.mark.parametrize("acc", [False, True], ids=["plain", "acc"])
+@pytest.mark.parametrize("layouts", ["kk", "tt", "gen"])
+def test_outer_product_is_rounded_once(hip, layouts, acc):
+    """K = 1 (the weight gradient of one token): every element is one float product,
+    with the bits numpy's float32 product has."""
+    M, N = 4096, 4100
+    announce(f"mul_mat outer product {layouts} {'acc' if acc else ''}")
+    rng = np.random.default_rng(17)
+    A, B = (rng.standard_normal((1, 1, r, 1)).astype(np.float32) for r in (M, N))
+    (ab, av), (bb, bv) = (laid(x, "gen" if layouts == "gen" else layouts[0]) for x in (A, B))
+    da, db, out = Dev(ab), Dev(bb), empty((1, 1, N, M))
+    (H.mul_mat_acc_f32 if acc else H.mul_mat_f32)(da.tensor(av), db.tensor(bv), out.tensor())
+    H.sync()
+    got = out.read()[0, 0]
+    for d in (da, db, out):
+        d.free()
+    assert np.array_equal(got, B[0, 0] * A[0, 0].T)
+
+
 # ---------------------------------------------------------------- strides of tens of megabytes
 
 @pytest.mark.parametrize("acc", [False, True], ids=["plain", "acc"])

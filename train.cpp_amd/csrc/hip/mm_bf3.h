@@ -9,8 +9,8 @@
 // Six v_mfma_f32_32x32x16_bf16 take 192 cycles of a SIMD for 32 x 32 x 16
 // products where v_mfma_f32_32x32x2_f32 takes 512 (and runs at the rate of the
 // vector ALU's FMAs). Error against 64 bits is below that of the FP32
-// instructions at every K measured, because a bf16 instruction rounds its
-// accumulator once per 16 k: rel 2-norm for normal inputs, FP32 -> here: K = 32
+// instructions from K = 2 on (K = 1 does not come here), because a bf16
+// instruction rounds its accumulator once per 16 k: rel 2-norm for normal inputs, FP32 -> here: K = 32
 // 1.05e-7 -> 0.40e-7, 128 1.95e-7 -> 0.64e-7, 1024 5.8e-7 -> 1.9e-7, 4096
 // 1.15e-6 -> 0.40e-6 (positive inputs at K = 4096 1.01e-6 -> 0.35e-6), and the
 // mean error is as near 0 (K = 4096: 2e-8 -> 5e-9 of the result's 2-norm).

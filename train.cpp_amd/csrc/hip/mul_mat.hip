@@ -631,8 +631,14 @@ int launch_mul_mat_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const t
     // them; the bf16 tiles are taken where their model's time is less (measured,
     // FP32 -> bf16: 768 x 2048 x 256 21.1 -> 19.1, 512 x 512 x 515 unaligned 24.6
     // -> 16.1; 512 x 512 x 512 15.1 -> 15.7, 300 x 300 x 300 11.0 -> 14.0).
+    // Up to 16 k always stay here: the bf16 tiles' slab would be half empty (K = 1, 4
+    // and 16, 4096 x 4096: 17.8 us here, 19.4 there; added to dst 25 and 27), and at
+    // K = 1 they round worse: leaving out the smallest partial products costs up to an
+    // ulp where the FP32 instruction's one product is rounded correctly (2-norm of the
+    // error 2.53e-8 here, 2.60e-8 there; from K = 2 on it is smaller there, 3.11e-8
+    // against 2.62e-8).
     const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * planes;
-    if (mm_bf3_fits(p)) {
+    if (p.K > 16 && mm_bf3_fits(p)) {
         // added into dst: K stays in one part
         B3Plan plan = mm_bf3_plan(p, planes, accumulate ? 1 : 8);
         const double slabs = (double) ((p.K + 31) / 32);
