@@ -241,8 +241,6 @@ __global__ __launch_bounds__(WI * WJ * 64) void k_mul_mat(MMArgs p) {
         // plus uniform multiples of nb1, and rows or columns past dst get an
         // offset past the resource (reads 0, stores dropped), so there is no
         // branch and each block's accumulators are read only when it is stored.
-        // (A column that is not there adds no multiple of nb1: 27 of them can
-        // pass 4 GiB, and the sum would be an offset into dst again.)
         const __amdgpu_buffer_rsrc_t rd =
             __builtin_amdgcn_make_buffer_rsrc((void*) d, (short) 0, (int) p.d_span, MM_RSRC_WORD3);
 #pragma unroll
@@ -268,17 +266,19 @@ __global__ __launch_bounds__(WI * WJ * 64) void k_mul_mat(MMArgs p) {
                 } else {  // the tile's last columns lie past dst: four at a time (fewer offsets held)
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        auto off = [&](int v) {
+#pragma unroll
+                        for (int v = 4 * q; v < 4 * q + 4; ++v) {
                             const int c = 8 * (v >> 2) + (v & 3);
-                            return vo != MM_OUT && jb + c < p.N ? vo + (uint32_t) (c * p.d_nb1) : MM_OUT;
-                        };
+                            old[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                                   rd, jb + c < p.N ? vo : MM_OUT, (uint32_t) (c * p.d_nb1), 0));
+                        }
 #pragma unroll
-                        for (int v = 4 * q; v < 4 * q + 4; ++v)
-                            old[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, off(v), 0, 0));
-#pragma unroll
-                        for (int v = 4 * q; v < 4 * q + 4; ++v)
+                        for (int v = 4 * q; v < 4 * q + 4; ++v) {
+                            const int c = 8 * (v >> 2) + (v & 3);
                             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, old[v] + acc[x][y][v]),
-                                                                  rd, off(v), 0, 0);
+                                                                  rd, jb + c < p.N ? vo : MM_OUT,
+                                                                  (uint32_t) (c * p.d_nb1), 0);
+                        }
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
@@ -624,6 +624,22 @@ int launch_mul_mat_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const t
         if (p.N <= 32) return launch_skinny_nt<2, 2>(s, sbm, planes, stream);
         if (p.N <= 48) return launch_skinny_nt<3, 2>(s, sbm, planes, stream);
         return launch_skinny_nt<4, 1>(s, sbm, planes, stream);
+    }
+
+    // Added to dst, a tile forms offsets for 28 columns whether they are there or not:
+    // where those pass 2 GiB (a few columns more than 79 MB apart), past which the sum
+    // with MM_OUT would be an offset into dst again, each column is a call of its own.
+    if (accumulate && p.N < 28 && 27 * p.d_nb1 > (int64_t) MM_PAST) {
+        trc_hip_tensor bc = b, dc = d;
+        bc.ne[1] = dc.ne[1] = 1;
+        dc.nb[1] = 4;  // of one column, not used
+        for (int64_t j = 0; j < p.N; ++j) {
+            bc.data = (uint8_t*) b.data + j * p.b_nb1;
+            dc.data = (uint8_t*) d.data + j * p.d_nb1;
+            const int rc = launch_mul_mat_f32(a, bc, dc, stream, true);
+            if (rc != TRC_HIP_OK) return rc;
+        }
+        return TRC_HIP_OK;
     }
 
     // Tiles of 64 x 64 with the FP32 instructions take 5 us and 0.7 us per 32 k
