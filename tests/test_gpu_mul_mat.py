@@ -742,6 +742,20 @@ def test_outer_product_is_rounded_once(hip, layouts, acc):
     assert np.array_equal(got, B[0, 0] * A[0, 0].T)
 
 
+@pytest.mark.parametrize("case", [
+    # (K, M, N, layouts, route): few slabs against one strided operand are faster on the
+    # FP32 tiles, many, or two such operands, on the bf16 tiles
+    (512, 1024, 1024, "gen,k", "fp32"), (512, 512, 512, "t,gen", "fp32"), (128, 2048, 2048, "gen,k", "fp32"),
+    (4096, 256, 256, "gen,k", "slots"), (1056, 1281, 1283, "gen,gen", "pair"), (512, 2048, 2048, "k,gen", "whole8"),
+])
+def test_strided_operands_choose_their_tiles(hip, case):
+    K, M, N, layouts, route = case
+    announce(f"mul_mat strided operands {case}")
+    A, B = synth.normal(990 + K, K * M).reshape(1, 1, M, K), synth.normal(991 + N, K * N).reshape(1, 1, N, K)
+    got = bf16_run(A, B, layouts.split(","), False, route)
+    assert _rel(got, _f64(A, B)) <= 2.0 ** -25 * np.sqrt(K)
+
+
 # ---------------------------------------------------------------- strides of tens of megabytes
 
 @pytest.mark.parametrize("acc", [False, True], ids=["plain", "acc"])

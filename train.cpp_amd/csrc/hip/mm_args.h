@@ -26,6 +26,10 @@ struct MMArgs {
     int part;           // the part of a launch that computes one of them
 };
 
+// operands that run along neither dimension: both kernels load these by element
+inline bool mm_a_strided(const MMArgs& p) { return p.a_nb0 != 4 && p.a_nb1 != 4; }
+inline bool mm_b_strided(const MMArgs& p) { return p.b_nb0 != 4 && p.b_nb1 != 4; }
+
 constexpr uint32_t MM_RSRC_WORD3 = 0x00020000u;  // gfx9 buffer resource: raw 32-bit dwords
 constexpr uint32_t MM_OUT = 0x80000000u;         // an offset past the resource: loads read 0, stores drop
 

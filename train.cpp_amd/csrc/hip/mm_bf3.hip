@@ -24,18 +24,27 @@ B3Plan mm_bf3_plan(const MMArgs& p, int64_t planes, int max_parts) {
     // 1.6 per part (16 to 64 tiles; two parts that meet in dst 12, six 17, eight
     // 19 to 24). 4096 x 4096 x 128, parts 1, 2, 3, 4, 6, 8: 107.6, 63.0, 45.5,
     // 38.9, 34.9, 39.2; 1024 x 1024 x 512: 32.3, 25.1, 20.6, 20.9, 21.9, 27.2.
+    // Operands that run along neither dimension load element by element, and with
+    // them the other operand: a slab takes 2.4 with one such operand, 3.3 with two,
+    // 0.6 of that where the last 64 columns are empty, and a launch that fills the
+    // chip 12 more (256 x 256 x 512 in two parts 35 and 42, 1408 x 1408 x 1024 60 and
+    // 74, 1408 x 1408 x 512 40 and 47); 3.5 where two workgroups share a CU and src0
+    // is strided (4096 x 4096 x 512 231, with src1 strided 150).
     const int64_t tiles = ((p.M + B3_T - 1) / B3_T) * ((p.N + B3_T - 1) / B3_T) * planes;
     const int64_t cus = device_cus();
     const double slabs = (double) ((p.K + 31) / 32);
-    const double slab = p.N <= 64 ? 0.7 : 0.8;
-    B3Plan best{2, 1, 7.5 + slab * slabs * (double) ((tiles + cus - 1) / cus)};
+    const bool sa = mm_a_strided(p), sb = mm_b_strided(p);
+    const bool narrow = p.N <= 64, strided = sa || sb;
+    const double slab = strided ? (sa && sb ? 3.3 : sa && tiles > cus ? 3.5 : 2.4) * (narrow ? 0.6 : 1) : narrow ? 0.7 : 0.8;
+    auto base = [&](int64_t groups) { return strided ? 12 * (groups < cus ? (double) groups / cus : 1.0) : 0; };
+    B3Plan best{2, 1, base(tiles) + 7.5 + slab * slabs * (double) ((tiles + cus - 1) / cus)};
     for (int parts = 2; parts <= max_parts; ++parts) {
         // a part is at least 4 slabs: shorter ones are all launch and meeting
         if (slabs < 4 * parts || tiles * parts > (parts == 2 ? 4 * cus : cus)) break;
         if (parts > 2 && tiles * parts > (int64_t) MM_SLOTS) break;
         if (tiles * 16 > MM_TICKETS) break;
         const double each = (double) (((int64_t) slabs + parts - 1) / parts);
-        const double us = 8 + 1.6 * parts + slab * each * (double) ((tiles * parts + cus - 1) / cus);
+        const double us = base(tiles * parts) + 8 + 1.6 * parts + slab * each * (double) ((tiles * parts + cus - 1) / cus);
         if (us < best.us) best = {2, parts, us};
     }
     // More tiles than CUs with K whole: 4-wave workgroups, two to a CU, whose
