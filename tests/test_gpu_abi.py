@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from conftest import announce
-from gpu_util import Dev, empty
+from gpu_util import Dev, empty, launches
 from traincpp_amd import hip as H
 
 pytestmark = pytest.mark.gpu
@@ -128,3 +128,29 @@ def test_cpy_permuted_planes(hip, shape, dtype):
         assert not got[..., view.shape[-1]:].any()
         out.free()
     src.free()
+
+
+@pytest.mark.parametrize("shape,turn,into,workgroups", [
+    # one 16-byte piece or element per lane: rows, and a transpose written into; tiles of
+    # 64 x 64
+    ((512, 64), False, True, 512 * 16 / 256), ((1001, 1000), True, True, 1001000 / 256),
+    ((13, 1000), True, False, 16),
+    ((64, 70), True, False, 2),
+])
+def test_cpy_work_per_lane(hip, shape, turn, into, workgroups):
+    announce(f"abi cpy work per lane {shape} {turn} {into}")
+    x = np.random.default_rng(33).standard_normal(shape).astype(np.float32)
+    view_of = lambda b: b.T if turn else b
+    if into:  # a contiguous src, dst the (transposed) view of a buffer
+        src, dst = Dev(np.ascontiguousarray(view_of(x))), empty(shape)
+        s, d = src.tensor(), dst.tensor(view_of(dst.base))
+    else:
+        src, dst = Dev(x), empty(view_of(x).shape)
+        s, d = src.tensor(view_of(src.base)), dst.tensor()
+    (grid, block), = launches(lambda stream: H.cpy(s, d, stream))
+    assert block == 256 and grid == -(-workgroups // 1)
+    H.cpy(s, d)
+    H.sync()
+    assert np.array_equal(dst.read(), x if into else view_of(x))
+    src.free()
+    dst.free()

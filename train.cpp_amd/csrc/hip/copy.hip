@@ -29,32 +29,25 @@ __global__ __launch_bounds__(CP_THREADS) void k_fill_f32x4(f4* __restrict__ dst,
 // (tensor_offset_linear, src/core/trc_tensor.cpp:95-103), ne0 fastest, so a run of
 // ne0 is one wave's contiguous read (or write) whenever that side has nb0 ==
 // element size. Rows that run along ne0 on both sides in whole aligned 16-byte
-// pieces are copied as such pieces. Bound by HBM; with 64-bit divisions per 4-byte
-// element the merge of 32 heads ([128, 512, 32, 4], 67 MB each way) took 30 us,
-// with four 16-byte pieces per lane in flight and 32-bit multiplies 11 (6.2 TB/s).
-constexpr int CP_ITEMS = 4;
+// pieces are copied as such pieces. Bound by HBM, and by the launch up to about a
+// megabyte; 64-bit divisions per 4-byte element took 30 us for the merge of 32 heads
+// ([128, 512, 32, 4], 67 MB each way), 16-byte pieces and 32-bit multiplies 11 (6.2
+// TB/s). One piece per lane: four took as long on large rows, 0.4 to 0.5 us more up
+// to a megabyte ([64, 512] 2.30 -> 2.79), and up to twice as long where dst does not
+// run along ne0 (1000 x 1001 written transposed 8.8 -> 16.9, [1000, 3, 500] 12.5 ->
+// 26.3; only an order of four reversed dimensions gained, 64 each 243 -> 171).
 template <typename T>
 __global__ __launch_bounds__(CP_THREADS) void k_cpy32(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
                                                      uint32_t total, FastDiv ne0, FastDiv ne1, FastDiv ne2,
                                                      int64_t snb0, int64_t snb1, int64_t snb2, int64_t snb3,
                                                      int64_t dnb0, int64_t dnb1, int64_t dnb2, int64_t dnb3) {
-    const uint32_t first = blockIdx.x * (CP_THREADS * CP_ITEMS) + threadIdx.x;
-    T v[CP_ITEMS];
-    int64_t to[CP_ITEMS];
-#pragma unroll
-    for (int k = 0; k < CP_ITEMS; ++k) {
-        const uint32_t idx = first + k * CP_THREADS;
-        if (idx >= total) continue;
-        const uint32_t r = div_by(idx, ne0), i0 = idx - r * ne0.d;
-        const uint32_t r2 = div_by(r, ne1), i1 = r - r2 * ne1.d;
-        const uint32_t i3 = div_by(r2, ne2), i2 = r2 - i3 * ne2.d;
-        v[k] = *(const T*) (src + i0 * snb0 + i1 * snb1 + i2 * snb2 + i3 * snb3);
-        to[k] = i0 * dnb0 + i1 * dnb1 + i2 * dnb2 + i3 * dnb3;
-    }
-#pragma unroll
-    for (int k = 0; k < CP_ITEMS; ++k) {
-        if (first + k * CP_THREADS < total) *(T*) (dst + to[k]) = v[k];
-    }
+    const uint32_t idx = blockIdx.x * CP_THREADS + threadIdx.x;
+    if (idx >= total) return;
+    const uint32_t r = div_by(idx, ne0), i0 = idx - r * ne0.d;
+    const uint32_t r2 = div_by(r, ne1), i1 = r - r2 * ne1.d;
+    const uint32_t i3 = div_by(r2, ne2), i2 = r2 - i3 * ne2.d;
+    *(T*) (dst + i0 * dnb0 + i1 * dnb1 + i2 * dnb2 + i3 * dnb3) =
+        *(const T*) (src + i0 * snb0 + i1 * snb1 + i2 * snb2 + i3 * snb3);
 }
 
 // The same for 2^31 elements and more.
@@ -194,7 +187,7 @@ int launch_cpy(const trc_hip_tensor& s, const trc_hip_tensor& d, size_t es, hipS
             return check_launch("cpy (transpose)");
         }
     }
-    if (n < ((int64_t) 1 << 31) - CP_THREADS * CP_ITEMS) {
+    if (n < ((int64_t) 1 << 31) - CP_THREADS) {
         // whole 16-byte pieces of rows that run along ne0 on both sides
         uintptr_t bits = (uintptr_t) sp | (uintptr_t) dp | (uintptr_t) (s.ne[0] * (int64_t) es);
         for (int k = 1; k < 4; ++k) {
@@ -205,7 +198,7 @@ int launch_cpy(const trc_hip_tensor& s, const trc_hip_tensor& d, size_t es, hipS
         const int64_t ne0 = s.ne[0] * (int64_t) es / (int64_t) w;
         const int64_t snb0 = w == 16 ? 16 : (int64_t) s.nb[0], dnb0 = w == 16 ? 16 : (int64_t) d.nb[0];
         const uint32_t total = (uint32_t) (ne0 * rows);
-        const dim3 grid((total + CP_THREADS * CP_ITEMS - 1) / (CP_THREADS * CP_ITEMS));
+        const dim3 grid((total + CP_THREADS - 1) / CP_THREADS);
 #define TRC_CPY32(T)                                                                                             \
     hipLaunchKernelGGL(k_cpy32<T>, grid, dim3(CP_THREADS), 0, stream, sp, dp, total, fast_div(ne0),              \
                        fast_div(s.ne[1]), fast_div(s.ne[2]), snb0, (int64_t) s.nb[1], (int64_t) s.nb[2],         \
