@@ -131,10 +131,10 @@ def test_cpy_permuted_planes(hip, shape, dtype):
 
 
 @pytest.mark.parametrize("shape,turn,into,workgroups", [
-    # one 16-byte piece or element per lane: rows, and a transpose written into; tiles of
-    # 64 x 64
+    # one 16-byte piece or element per lane: rows, a transpose written into, and few
+    # transposed runs; from 13 runs on, tiles of 64 x 64
     ((512, 64), False, True, 512 * 16 / 256), ((1001, 1000), True, True, 1001000 / 256),
-    ((13, 1000), True, False, 16),
+    ((2, 5000), True, False, 10000 / 256), ((12, 1000), True, False, 12000 / 256), ((13, 1000), True, False, 16),
     ((64, 70), True, False, 2),
 ])
 def test_cpy_work_per_lane(hip, shape, turn, into, workgroups):
