@@ -9,7 +9,7 @@ import pytest
 
 import oracle_lib as O
 from conftest import announce
-from gpu_util import Dev, Stream, empty, mem_free
+from gpu_util import Dev, Stream, empty, launches, mem_free
 from test_oracle_dequant import TYPES
 from traincpp_amd import hip as H
 from traincpp_amd import synth
@@ -483,3 +483,22 @@ def test_two_slices_of_columns(hip, name, K, M, N):
     assert np.array_equal(dy.read().view(np.uint32), got.view(np.uint32))
     for d in (dw, dx, dy):
         d.free()
+
+
+@pytest.mark.parametrize("M,N,calls", [(8192, 33, 1), (8192, 64, 1), (8193, 48, 2), (8193, 64, 2), (9000, 49, 2),
+                                       (11264, 64, 2), (11265, 49, 1), (14336, 64, 1), (14336, 48, 2)])
+def test_slices_in_one_call_or_two(hip, M, N, calls):
+    """One call for both slices of 32 columns where it needs no second round of
+    workgroups, or fills that; else a call for each: launches of the pre-pass and the
+    product on a device of 256 CUs (a call for 16 columns or fewer may convert x itself)."""
+    K, t = 512, TYPES["q4_0"]
+    announce(f"qmatvec slices M={M} N={N}")
+    raw = synth.block_bytes(synth.quant_blocks(t, K * M // 32, 975))
+    X = synth.normal(976 + N, K * N).reshape(1, 1, N, K)
+    dw, dx, dy = Dev(raw), Dev(X), empty((1, 1, N, M))
+    args = (t, dw.ptr, K, M, (K // 32) * H.BLOCK_BYTES[t], dx.ptr, N, K * 4, dy.ptr, M * 4)
+    got = launches(lambda s: H.qmatvec(*args, s))
+    assert (len(got) == 2) == (calls == 1)
+    for d in (dw, dx, dy):
+        d.free()
+    assert O.row_l2_error(gpu_qmatvec(t, raw, K, M, X), oracle_qmatvec(t, raw, K, M, X)) <= TOL

@@ -1513,12 +1513,15 @@ int launch_type(const void* wq, int64_t K, int64_t M, size_t nb1_w, const float*
 
 int launch_qmatvec(int type, const void* wq, int64_t K, int64_t M, size_t nb1_w, const float* x, int64_t N,
                    size_t nb1_x, float* y, size_t nb1_y, hipStream_t stream, QmScratch where) {
-    // Two slices of 32 columns go in one call of the matrix-core kernel, unless M
-    // fills the chip with one slice and the second is at most half full: then a call
-    // for 32 columns and a narrower one for the rest take less (Q4_0, K = 4096, M =
-    // 14336, one call against two: N = 33 33.8 / 28.4 us, 40 33.3 / 32.3, 48 33.5 /
-    // 33.6, 64 33.8 / 39.0; K = 11008, M = 4096: N = 33 27.3 / 31.2, 50 27.6 / 41.0).
-    const bool slices = N > 48 || (N > 32 && M <= 32 * (int64_t) device_cus());
+    // Two slices of 32 columns go in one call of the matrix-core kernel, unless that
+    // takes a second round of workgroups (64 rows each at most) that two calls, of 40 to
+    // 64 rows each, spare: always where the second slice is at most half full, otherwise
+    // while the second round is under half full too (one call against two, K = 4096, Q4_0:
+    // M = 14336 N = 33 33.8 / 28.4 us, 48 33.5 / 33.6, 64 33.8 / 39.0; M = 9000 N = 64 33.2
+    // / 30.7, Q5_1 46.8 / 41.9, Q8_0 39.7 / 35.9; M = 11008 33.0 / 30.8, 46.7 / 43.6, 39.0 /
+    // 38.9; M = 12288 32.0 / 31.5, 46.2 / 44.4, 37.5 / 40.4; K = 11008, M = 4096: N = 33 27.3
+    // / 31.2, 50 27.6 / 41.0).
+    const bool slices = N > 32 && (M <= 32 * (int64_t) device_cus() || (N > 48 && M > 44 * (int64_t) device_cus()));
     if (N > 16 && !((N <= 32 || slices) && qmm_supported(K, N, wq, nb1_w))) {
         // skinny GEMM beyond the columns one launch carries: one fused pass over W
         // per 32 columns on the matrix-core kernel, else per 16 (the launches run
