@@ -11,7 +11,7 @@ import pytest
 
 import oracle_lib as O
 from conftest import announce
-from gpu_util import Dev, empty
+from gpu_util import Dev, empty, mem_free
 from traincpp_amd import hip as H
 
 pytestmark = pytest.mark.gpu
@@ -542,3 +542,22 @@ def test_acc_regions_bitwise(hip, bshape, pads, offset):
     assert np.array_equal(da.read().view(np.uint32), want.view(np.uint32))
     da.free()
     db.free()
+
+
+@pytest.mark.parametrize("n", [(1 << 33) + 1, (1 << 34) - 1024, (1 << 34) + 5])
+def test_contiguous_elementwise_past_one_launch(hip, n):
+    """Tensors of 32 GiB and more, where four floats per thread pass half of the 2^32
+    threads of one launch, and all of them: every part is scaled, in place."""
+    if mem_free() < 4 * n + (4 << 30):
+        pytest.skip("needs 68 GiB of free device memory")
+    announce(f"scale {n} floats in place")
+    buf = H.DeviceBuffer(4 * n)
+    H.fill_f32(buf.ptr, 1.25, n)
+    t = H.tensor(buf.ptr, [n, 1, 1, 1], [4, 4 * n, 4 * n, 4 * n])
+    H.scale_f32(t, t, 2.0)
+    H.sync()
+    part = np.empty(1 << 16, np.float32)
+    for at in [0, n // 3, n // 2, (1 << 32) - 100, (1 << 33) - part.size, n - part.size]:
+        H.check(H.load().trc_hip_d2h(part.ctypes.data, buf.ptr + 4 * at, part.nbytes, None))
+        assert np.all(part == 2.5)
+    buf.free()

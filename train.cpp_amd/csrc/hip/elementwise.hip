@@ -871,20 +871,27 @@ bool shape_ok(const trc_hip_tensor& t) {
 
 bool flat_f32(const trc_hip_tensor& t) { return (((uintptr_t) t.data) & 15u) == 0 && contiguous_f32(t); }
 
+// A launch runs under 2^32 threads (HIP drops the rest without a word): FLAT_MAX floats
+// at a time.
+constexpr int64_t FLAT_MAX = (int64_t) 1 << 33;
 template <FlatOp OP>
 int launch_flat(const char* name, const void* a, const void* b, void* d, int64_t n, float scale, hipStream_t s) {
-    const int64_t blocks = (n / 4 + EW_THREADS) / EW_THREADS;  // one more float4 for the tail
-    if (n >= FLAT_NT) {
-        hipLaunchKernelGGL((k_flat<OP, true>), dim3((unsigned) blocks), dim3(EW_THREADS), 0, s, (const f4*) a,
-                           (const f4*) b, (f4*) d, n, scale);
-    } else {
-        hipLaunchKernelGGL((k_flat<OP, false>), dim3((unsigned) blocks), dim3(EW_THREADS), 0, s, (const f4*) a,
-                           (const f4*) b, (f4*) d, n, scale);
+    for (int64_t at = 0; at < n; at += FLAT_MAX) {
+        const int64_t m = n - at < FLAT_MAX ? n - at : FLAT_MAX;
+        const int64_t blocks = (m / 4 + EW_THREADS) / EW_THREADS;  // one more float4 for the tail
+        const f4* fa = (const f4*) ((const float*) a + at);
+        const f4* fb = b != nullptr ? (const f4*) ((const float*) b + at) : nullptr;
+        f4* fd = (f4*) ((float*) d + at);
+        if (n >= FLAT_NT) {
+            hipLaunchKernelGGL((k_flat<OP, true>), dim3((unsigned) blocks), dim3(EW_THREADS), 0, s, fa, fb, fd, m, scale);
+        } else {
+            hipLaunchKernelGGL((k_flat<OP, false>), dim3((unsigned) blocks), dim3(EW_THREADS), 0, s, fa, fb, fd, m, scale);
+        }
+        const int rc = check_launch(name);
+        if (rc != TRC_HIP_OK) return rc;
     }
-    return check_launch(name);
+    return TRC_HIP_OK;
 }
-// grids past one launch's 2^31 workgroups stay with the row kernels
-bool flat_fits(int64_t n) { return n / 4 / EW_THREADS < 0x7FFFFFFF; }
 
 template <BinOp OP>
 int launch_binary(const char* name, const trc_hip_tensor& a, const trc_hip_tensor& b, const trc_hip_tensor& d,
@@ -899,7 +906,7 @@ int launch_binary(const char* name, const trc_hip_tensor& a, const trc_hip_tenso
         }
     }
     if (!f32_aligned(a) || !f32_aligned(b) || !f32_aligned(d)) return fail(TRC_HIP_E_ALIGN, "%s: 4-byte alignment", name);
-    if (flat_f32(a) && flat_f32(d) && flat_f32(b) && nelem(a) == nelem(b) && flat_fits(nelem(d))) {
+    if (flat_f32(a) && flat_f32(d) && flat_f32(b) && nelem(a) == nelem(b)) {
         return launch_flat<OP == BinOp::ADD ? FlatOp::ADD : FlatOp::MUL>(name, a.data, b.data, d.data, nelem(d), 0.f, s);
     }
     const int64_t rows = d.ne[1] * d.ne[2] * d.ne[3];
@@ -933,7 +940,7 @@ int launch_unary(const char* name, const trc_hip_tensor& a, const trc_hip_tensor
         if (d.ne[k] != a.ne[k]) return fail(TRC_HIP_E_SHAPE, "%s: dst must have a's shape (dim %d)", name, k);
     }
     if (!f32_aligned(a) || !f32_aligned(d)) return fail(TRC_HIP_E_ALIGN, "%s: 4-byte alignment", name);
-    if (flat_f32(a) && flat_f32(d) && flat_fits(nelem(d))) {
+    if (flat_f32(a) && flat_f32(d)) {
         return launch_flat<OP == UnOp::SQR ? FlatOp::SQR : FlatOp::SCALE>(name, a.data, nullptr, d.data, nelem(d), scale, s);
     }
     const int64_t rows = d.ne[1] * d.ne[2] * d.ne[3];
@@ -1097,7 +1104,7 @@ int launch_acc_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const trc_h
     // a region as dense as b: one run of floats
     if (flat_f32(b) && ((((uintptr_t) d.data) | offset) & 15u) == 0 && (b.ne[1] == 1 || nb1 == (size_t) b.ne[0] * 4) &&
         (b.ne[2] == 1 || nb2 == (size_t) (b.ne[0] * b.ne[1]) * 4) &&
-        (b.ne[3] == 1 || nb3 == (size_t) (b.ne[0] * b.ne[1] * b.ne[2]) * 4) && flat_fits(nelem(b))) {
+        (b.ne[3] == 1 || nb3 == (size_t) (b.ne[0] * b.ne[1] * b.ne[2]) * 4)) {
         uint8_t* at = (uint8_t*) d.data + offset;
         return launch_flat<FlatOp::ADD>("acc", at, b.data, at, nelem(b), 0.f, s);
     }
