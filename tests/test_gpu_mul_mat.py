@@ -488,15 +488,15 @@ def test_bf16_tiles_against_float64(hip, shape, layout):
 
 
 # one shape per way the parts of K come together: K whole on 8-wave and 4-wave
-# workgroups, two parts in dst, more in slots
-BF16_ROUTES = [(640, 1024, 512, 2), (128, 2048, 512, 8), (1024, 2048, 1024, 1), (4096, 512, 200, 1)]
+# workgroups, two parts in dst, more in slots (of one and of two planes)
+BF16_ROUTES = [((1024, 2560, 1280, 1), "whole8"), ((128, 2048, 512, 8), "whole4"), ((1024, 2048, 1024, 1), "pair"),
+               ((4096, 512, 200, 1), "slots"), ((640, 1024, 512, 2), "slots")]
 
 
-@pytest.mark.parametrize("shape", BF16_ROUTES)
-def test_bf16_tiles_special_values(hip, shape):
+@pytest.mark.parametrize("shape,route", BF16_ROUTES)
+def test_bf16_tiles_special_values(hip, shape, route):
     """Infinities, NaNs, values that round to infinity as bf16, subnormals and values
-    whose last bits bf16 cannot hold, each in rows and columns of their own: results
-    are float64's (not finite where it is not, equal to float rounding elsewhere), and
+    near them, each in rows and columns of their own: results are float64's (not finite where it is not, equal to float rounding elsewhere), and
     the other rows' bits are what they are without them, in tiles that hold none."""
     K, M, N, P = shape
     rng = np.random.default_rng(7 * K + M)
@@ -517,6 +517,9 @@ def test_bf16_tiles_special_values(hip, shape):
     B[0, 0, 9, 0] = -np.inf
     clean[1][0, 0, 9] = B[0, 0, 9]
     da, db, dc = Dev(A), Dev(B), Dev(clean[0])
+    out = empty((1, P, N, M))
+    assert bf16_route(da.tensor(), db.tensor(), out.tensor()) == route
+    out.free()
     got = gpu_mul_mat(da, A, db, B)
     plain = gpu_mul_mat(dc, clean[0], db, B)
     with np.errstate(invalid="ignore", over="ignore"):
@@ -537,8 +540,8 @@ def test_bf16_tiles_special_values(hip, shape):
         d.free()
 
 
-@pytest.mark.parametrize("shape", BF16_ROUTES)
-def test_bf16_tiles_integers_are_exact(hip, shape):
+@pytest.mark.parametrize("shape,route", BF16_ROUTES)
+def test_bf16_tiles_integers_are_exact(hip, shape, route):
     """Integer operands whose sums stay under 2^24: every sum is exact in float, so
     the bits are those of any order of adding."""
     K, M, N, P = shape
@@ -548,7 +551,9 @@ def test_bf16_tiles_integers_are_exact(hip, shape):
     B = rng.integers(-60, 61, (1, P, N, K)).astype(np.float32)
     A[0, 0, 0], B[0, 0, 0] = 0, 0
     A[0, 0, 0, K // 3], B[0, 0, 0, K // 3] = 1, 16777215.0
-    da, db = Dev(A), Dev(B)
+    da, db, out = Dev(A), Dev(B), empty((1, P, N, M))
+    assert bf16_route(da.tensor(), db.tensor(), out.tensor()) == route
+    out.free()
     got = gpu_mul_mat(da, A, db, B)
     da.free()
     db.free()
@@ -679,14 +684,14 @@ def laid(x, layout):
     return base, view
 
 
-def bf16_run(A, B, layouts, acc, route):
-    """The product (added into zeros where acc) of A and B laid out as given, whose
-    launch is asserted to be `route`."""
+def bf16_run(A, B, layouts, acc, route, D=None):
+    """The product (added into D, or into zeros, where acc) of A and B laid out as
+    given, whose launch is asserted to be `route`."""
     (ab, av), (bb, bv) = laid(A, layouts[0]), laid(B, layouts[1])
     da, db, out = Dev(ab), Dev(bb), empty((1, B.shape[1], B.shape[2], A.shape[2]))
     ta, tb, td = da.tensor(av), db.tensor(bv), out.tensor()
     assert bf16_route(ta, tb, td, acc) == route
-    H.fill_f32(out.ptr, 0.0, out.base.size)
+    out.buf.upload(out.base if D is None else D)
     (H.mul_mat_acc_f32 if acc else H.mul_mat_f32)(ta, tb, td)
     H.sync()
     got = out.read()
@@ -698,6 +703,60 @@ def bf16_run(A, B, layouts, acc, route):
 # (K, M, N, accumulated, route): one shape for each way the parts of K come together
 BF16_ONE_EACH = [(1056, 1409, 1410, False, "whole8"), (200, 2689, 2690, False, "whole4"), (1000, 1409, 1411, True, "whole8"),
                  (200, 2691, 2689, True, "whole4"), (1056, 1281, 1283, False, "pair"), (1056, 777, 130, False, "slots")]
+
+
+@pytest.mark.parametrize("layouts", ["k,k", "t,k", "k,t", "t,t", "odd,odd", "gen,gen"])
+@pytest.mark.parametrize("shape", BF16_ONE_EACH)
+def test_bf16_tiles_not_finite(hip, shape, layouts):
+    """The second pass, with the FP32 instructions, that a tile makes for a result that
+    is not finite on the bf16 ones: in the first and the last rows and columns of tiles,
+    with a last slab that is not whole, a last column tile under half full, every
+    loader, and added to dst. Infinities, NaNs, operands from 2^104 and sums from 2^80
+    on come out as float64's within K float roundings; tiles without any keep their bits."""
+    K, M, N, acc, route = shape
+    announce(f"mul_mat bf16 tiles not finite {shape} {layouts}")
+    rng = np.random.default_rng(K + 3 * M)
+    A, B, D = (rng.standard_normal((1, 1, r, c)).astype(np.float32) for r, c in ((M, K), (N, K), (N, M)))
+    B[..., K // 2] = np.clip(B[..., K // 2], -0.9, 0.9)
+    plain = bf16_run(A, B, layouts.split(","), acc, route, D)
+    for i in (0, M - 8):
+        A[0, 0, i, 5] = np.inf
+        A[0, 0, i + 1, K - 1] = np.nan
+        A[0, 0, i + 2] = 0
+        A[0, 0, i + 2, K // 2] = 3.4e38                # infinity as bf16; finite times the column above
+        A[0, 0, i + 3, K - 2] = -1e32                  # infinity times 2^24
+        A[0, 0, i + 4] *= np.float32(1e25)
+        A[0, 0, i + 5] *= np.float32(1e-41)
+    B[0, 0, N - 1, 3] = -np.inf
+    got = bf16_run(A, B, layouts.split(","), acc, route, D)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = _f64(A, B) + (D if acc else 0)
+        w32 = want.astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(w32))
+    assert np.array_equal(got[np.isinf(w32)], w32[np.isinf(w32)])
+    ok = np.isfinite(w32)
+    a, b = (np.abs(np.nan_to_num(x, posinf=0, neginf=0).astype(np.float64)) for x in (A, B))
+    # K additions of half an ulp each (and the one into dst), and half the smallest subnormal for each
+    bound = K * (2.0 ** -24 * _f64(a, b) + 2.0 ** -150) + (2.0 ** -24 * np.abs(D) if acc else 0)
+    assert np.all(np.abs(got[ok].astype(np.float64) - want[ok]) <= bound[ok])
+    mid = (slice(None), slice(None), slice(0, (N - 1) // 128 * 128), slice(128, (M - 8) // 128 * 128))
+    assert got[mid].size and np.array_equal(got[mid].view(np.uint32), plain[mid].view(np.uint32))
+
+
+def test_bf16_tiles_long_sums_do_not_drift(hip):
+    """16384 positive products in one part of K: the error of K / 16 roundings of half an
+    ulp at most, which add up like a random walk (2-norm under sqrt(K / 16) half ulps),
+    and not in one direction (a loss of a hundredth of each rounding would move the mean
+    by 2^-24 K / 16 / 100 / 2, 5 half ulps)."""
+    K, M, N = 16384, 1409, 1410
+    announce("mul_mat bf16 tiles long positive sums")
+    rng = np.random.default_rng(23)
+    A, B = (rng.random((1, 1, r, K), dtype=np.float32) for r in (M, N))
+    got = bf16_run(A, B, "kk", True, "whole8")[:, :, -200:, -200:]
+    want = _f64(A[:, :, -200:], B[:, :, -200:])
+    err = got - want
+    assert np.linalg.norm(err) / np.linalg.norm(want) <= 2.0 ** -24 * np.sqrt(K / 16)
+    assert abs(err.mean()) / want.mean() <= 4 * 2.0 ** -24
 
 
 @pytest.mark.parametrize("layouts", ["kk", "tt"])
