@@ -10,7 +10,7 @@ import pytest
 
 import oracle_lib as O
 from conftest import GOLDEN, announce
-from gpu_util import Dev, empty
+from gpu_util import Dev, empty, mem_free
 from test_oracle_dequant import BYTES, M_SET, TYPES, pack_blocks, q_patterns
 from traincpp_amd import hip as H
 from traincpp_amd import synth
@@ -134,3 +134,27 @@ def test_misaligned_and_bad_type_are_rejected(hip):
     with pytest.raises(H.HipError) as e:
         H.dequant(12, src.ptr, 4, dst.ptr)  # Q4_K: not a legacy format
     assert e.value.code == H.E_INVALID
+
+
+@pytest.mark.parametrize("n_blocks", [(1 << 28) + 5, (1 << 29) + 5])
+def test_more_blocks_than_one_launch_takes(hip, n_blocks):
+    """Tensors of 32 and 64 GiB of floats, past the launch of 2^28 blocks and past 2^32
+    threads: blocks of equal bytes, looked at around the launches' ends."""
+    t = TYPES["q4_0"]
+    if mem_free() < n_blocks * (H.BLOCK_BYTES[t] + 128) + (4 << 30):
+        pytest.skip("needs 80 GiB of free device memory")
+    announce(f"dequant {n_blocks} blocks")
+    raw = np.full(H.BLOCK_BYTES[t], 0x3C, np.uint8)
+    want = O.dequant(t, raw)
+    src, dst = H.DeviceBuffer(n_blocks * raw.size), H.DeviceBuffer(n_blocks * 128)
+    H.check(H.load().trc_hip_memset(src.ptr, 0x3C, src.nbytes, None))
+    H.fill_f32(dst.ptr, float("nan"), n_blocks * 32)
+    H.dequant(t, src.ptr, n_blocks, dst.ptr)
+    H.sync()
+    part = np.empty((8, 32), np.float32)
+    for at in [0, (1 << 28) - 4, (1 << 29) - 4, n_blocks // 3, n_blocks - 8]:
+        if at + 8 <= n_blocks:
+            H.check(H.load().trc_hip_d2h(part.ctypes.data, dst.ptr + 128 * at, part.nbytes, None))
+            assert np.array_equal(part.view(np.uint32), np.tile(want.reshape(1, 32), (8, 1)).view(np.uint32))
+    src.free()
+    dst.free()

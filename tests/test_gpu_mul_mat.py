@@ -863,3 +863,43 @@ def test_operand_rows_far_apart(hip):
     for x in (buf, db, out):
         x.free()
     assert O.row_l2_error(got, O.mul_mat(t01(A[None, None]), B, threads=8)) <= TOL
+
+
+# ---------------------------------------------------------------- more workgroups than a launch takes
+
+@pytest.mark.parametrize("case", [
+    # (K, M, N, src0 planes, src1 planes): the few-column kernel's limit of 4.2 million
+    # workgroups and the tiles' of 16.8 million, the planes along either dimension
+    (4, 1, 1, (2, 3), (700000, 6)), (4, 1, 1, (1, 2), (1, 4200002)), (4, 1, 3, (1, 5000000), (1, 5000000)),
+    (1, 1, 1, (2, 3), (2800000, 6)), (1, 1, 1, (1, 1), (1, 16777300)), (1, 1, 1, (8400000, 1), (8400000, 2)),
+])
+@pytest.mark.parametrize("acc", [False, True], ids=["plain", "acc"])
+def test_more_planes_than_one_launch_takes(hip, case, acc):
+    K, M, N, (a3, a2), (b3, b2) = case
+    announce(f"mul_mat planes past one launch {case}")
+    rng = np.random.default_rng(K + b3)
+    A = rng.integers(-8, 9, (a3, a2, M, K)).astype(np.float32)
+    B = rng.integers(-8, 9, (b3, b2, N, K)).astype(np.float32)
+    D = rng.integers(-8, 9, (b3, b2, N, M)).astype(np.float32)
+    da, db, out = Dev(A), Dev(B), Dev(D)
+    (H.mul_mat_acc_f32 if acc else H.mul_mat_f32)(da.tensor(), db.tensor(), out.tensor())
+    H.sync()
+    got = out.read()
+    for d in (da, db, out):
+        d.free()
+    want = (B[..., :, None, :] * np.tile(A, (b3 // a3, b2 // a2, 1, 1))[..., None, :, :]).sum(-1)
+    assert np.array_equal(got, want + D if acc else want)
+
+
+def test_more_rows_than_one_launch_takes(hip):
+    """A src0 of 67.2 million rows of 4: 4.2 million workgroups of 16 rows."""
+    K, M, N = 4, 67_200_000, 2
+    announce(f"mul_mat rows past one launch {M}")
+    rng = np.random.default_rng(29)
+    A = rng.integers(-8, 9, (1, 1, M, K), dtype=np.int8).astype(np.float32)
+    B = rng.integers(-8, 9, (1, 1, N, K)).astype(np.float32)
+    da, db = Dev(A), Dev(B)
+    got = gpu_mul_mat(da, A, db, B)
+    da.free()
+    db.free()
+    assert np.array_equal(got[0, 0], B[0, 0] @ A[0, 0].T)

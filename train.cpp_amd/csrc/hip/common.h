@@ -111,6 +111,10 @@ __device__ __forceinline__ uint32_t div_by(uint32_t n, FastDiv f) {
     return (uint32_t) (((uint64_t) __umulhi(n, f.m) + n) >> f.s);
 }
 
+// HIP runs under 2^32 threads of a launch along one dimension, and drops the rest of a
+// larger one without an error.
+constexpr int64_t max_groups(int64_t threads) { return (((int64_t) 1 << 32) - 1) / threads; }
+
 // Launch-side error reporting, implemented in abi.hip.
 int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);

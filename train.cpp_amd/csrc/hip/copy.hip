@@ -176,13 +176,13 @@ int launch_cpy(const trc_hip_tensor& s, const trc_hip_tensor& d, size_t es, hipS
         const bool whole = s.ne[0] % TT == 0 && s.ne[1] % TT == 0 && (((uintptr_t) sp | (uintptr_t) dp) & 15u) == 0 &&
                            s.nb[0] % 16 == 0 && d.nb[1] % 16 == 0 && s.nb[2] % 16 == 0 && s.nb[3] % 16 == 0 &&
                            d.nb[2] % 16 == 0 && d.nb[3] % 16 == 0;
-        if (grid <= 0x7FFFFFFF && whole) {
+        if (grid <= max_groups(CP_THREADS) && whole) {
             hipLaunchKernelGGL(k_cpy_transpose4, dim3((unsigned) grid), dim3(CP_THREADS), 0, stream, sp, dp, s.ne[2],
                                tiles0, tiles1, (int64_t) s.nb[0], (int64_t) s.nb[2], (int64_t) s.nb[3],
                                (int64_t) d.nb[1], (int64_t) d.nb[2], (int64_t) d.nb[3]);
             return check_launch("cpy (transpose)");
         }
-        if (grid <= 0x7FFFFFFF) {
+        if (grid <= max_groups(CP_THREADS)) {
             hipLaunchKernelGGL(k_cpy_transpose, dim3((unsigned) grid), dim3(CP_THREADS), 0, stream, sp, dp, s.ne[0],
                                s.ne[1], s.ne[2], tiles0, tiles1, (int64_t) s.nb[0], (int64_t) s.nb[2],
                                (int64_t) s.nb[3], (int64_t) d.nb[1], (int64_t) d.nb[2], (int64_t) d.nb[3]);

@@ -131,12 +131,17 @@ __global__ __launch_bounds__(DQ_THREADS) void k_dequant(const uint8_t* __restric
 template <int TYPE>
 int launch_type(const void* blocks, int64_t n_blocks, float* dst, hipStream_t stream) {
     constexpr int ITEMS = 1;
-    const int64_t n_quads = n_blocks * 8;
-    const int64_t grid = (n_quads + ITEMS * DQ_THREADS - 1) / (ITEMS * DQ_THREADS);
-    if (grid > 0x7FFFFFFF) return fail(TRC_HIP_E_INVALID, "dequant: %lld blocks exceed one launch", (long long) n_blocks);
-    hipLaunchKernelGGL((k_dequant<TYPE, ITEMS>), dim3((unsigned) grid), dim3(DQ_THREADS), 0, stream,
-                       (const uint8_t*) blocks, n_quads, (f4*) dst);
-    return check_launch("dequant");
+    constexpr int64_t MAX_BLOCKS = (int64_t) 1 << 28;  // of a launch: 32 GiB of floats
+    static_assert(MAX_BLOCKS * 8 / (ITEMS * DQ_THREADS) < max_groups(DQ_THREADS), "under 2^32 threads");
+    for (int64_t at = 0; at < n_blocks; at += MAX_BLOCKS) {
+        const int64_t n_quads = (n_blocks - at < MAX_BLOCKS ? n_blocks - at : MAX_BLOCKS) * 8;
+        const int64_t grid = (n_quads + ITEMS * DQ_THREADS - 1) / (ITEMS * DQ_THREADS);
+        hipLaunchKernelGGL((k_dequant<TYPE, ITEMS>), dim3((unsigned) grid), dim3(DQ_THREADS), 0, stream,
+                           (const uint8_t*) blocks + at * block_bytes(TYPE), n_quads, (f4*) dst + at * 8);
+        const int rc = check_launch("dequant");
+        if (rc != TRC_HIP_OK) return rc;
+    }
+    return TRC_HIP_OK;
 }
 
 }  // namespace

@@ -871,9 +871,8 @@ bool shape_ok(const trc_hip_tensor& t) {
 
 bool flat_f32(const trc_hip_tensor& t) { return (((uintptr_t) t.data) & 15u) == 0 && contiguous_f32(t); }
 
-// A launch runs under 2^32 threads (HIP drops the rest without a word): FLAT_MAX floats
-// at a time.
-constexpr int64_t FLAT_MAX = (int64_t) 1 << 33;
+constexpr int64_t FLAT_MAX = (int64_t) 1 << 33;  // floats of a launch
+static_assert(FLAT_MAX / 4 / EW_THREADS < max_groups(EW_THREADS), "under 2^32 threads");
 template <FlatOp OP>
 int launch_flat(const char* name, const void* a, const void* b, void* d, int64_t n, float scale, hipStream_t s) {
     for (int64_t at = 0; at < n; at += FLAT_MAX) {

@@ -59,7 +59,7 @@ int launch_mm_bf3(MMArgs& p, int64_t planes, int groups, int parts, bool acc, hi
     p.tiles_j = (p.N + B3_T - 1) / B3_T;
     p.xcd_planes = planes % 8 == 0 ? 1 : 0;
     const int64_t tiles = p.tiles_i * p.tiles_j * planes;
-    if (tiles * parts > 0x7FFFFFFF) {
+    if (tiles * parts > max_groups(256 * groups)) {
         return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) tiles * parts);
     }
     const unsigned n = (unsigned) tiles;

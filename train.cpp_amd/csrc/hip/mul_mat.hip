@@ -522,7 +522,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void k_mm_skinny(SkArgs p) {
 template <int NT, int AHEAD>
 int launch_skinny_nt(SkArgs& p, int bmode, int64_t planes, hipStream_t stream) {
     const int64_t grid = p.row_blocks * planes;
-    if (grid > 0x7FFFFFFF) return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) grid);
+    if (grid > max_groups(SK_WAVES * 64)) return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) grid);
     if (NT == 1 && bmode == K_CONTIG && p.N > 4 && p.N <= 8) {
         // 5..8 columns: X in full lines (at 4 or fewer the 16-column loads are as fast)
         hipLaunchKernelGGL((k_mm_skinny<1, AHEAD, SK_X8>), dim3((unsigned) grid), dim3(SK_WAVES * 64), 0, stream, p);
@@ -553,7 +553,7 @@ int launch_cfg(MMArgs& p, int64_t planes, hipStream_t stream) {
     p.tiles_i = (p.M + BM - 1) / BM;
     p.tiles_j = (p.N + BN - 1) / BN;
     const int64_t grid = p.tiles_i * p.tiles_j * planes;
-    if (grid > 0x7FFFFFFF) return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) grid);
+    if (grid > max_groups(WI * WJ * 64)) return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) grid);
     p.xcd_planes = planes % 8 == 0 ? 1 : 0;
     p.d_span = (p.M - 1) * p.d_nb0 + (p.N - 1) * p.d_nb1 + 4;
     hipLaunchKernelGGL((k_mul_mat<WI, WJ, TI, TJ, BK, AM, BMO, ACC>), dim3((unsigned) grid),
@@ -579,6 +579,44 @@ int dispatch_modes(MMArgs& p, int am, int bm, int64_t planes, hipStream_t s) {
 }
 
 }  // namespace
+
+// The product in calls of as many planes, or of as many rows of one plane, as `groups`
+// workgroups carry, where a plane takes `per`.
+static int mul_mat_in_pieces(const trc_hip_tensor& a, const trc_hip_tensor& b, const trc_hip_tensor& d, int64_t per,
+                             int64_t groups, hipStream_t stream, bool accumulate) {
+    trc_hip_tensor pa = a, pb = b, pd = d;
+    const int k = b.ne[3] > 1 ? 3 : 2;
+    const int64_t unit = k == 3 ? per * b.ne[2] : per;
+    int64_t step;
+    if (b.ne[k] > 1) {
+        // whole periods of a's broadcast planes, or a part of one
+        step = groups / unit > 1 ? groups / unit : 1;
+        if (step > a.ne[k]) step -= step % a.ne[k];
+        for (int64_t at = 0, n; at < b.ne[k]; at += n) {
+            n = b.ne[k] - at < step ? b.ne[k] - at : step;
+            const int64_t first = at % a.ne[k];
+            if (step < a.ne[k] && n > a.ne[k] - first) n = a.ne[k] - first;
+            pa.ne[k] = n < a.ne[k] ? n : a.ne[k];
+            pb.ne[k] = pd.ne[k] = n;
+            pa.data = (uint8_t*) a.data + first * (int64_t) a.nb[k];
+            pb.data = (uint8_t*) b.data + at * (int64_t) b.nb[k];
+            pd.data = (uint8_t*) d.data + at * (int64_t) d.nb[k];
+            const int rc = launch_mul_mat_f32(pa, pb, pd, stream, accumulate);
+            if (rc != TRC_HIP_OK) return rc;
+        }
+        return TRC_HIP_OK;
+    }
+    step = (int64_t) ((double) a.ne[1] * (double) groups / (double) per / 2) / 128 * 128;
+    if (step == 0) return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) per);
+    for (int64_t at = 0; at < a.ne[1]; at += step) {
+        pa.ne[1] = pd.ne[0] = a.ne[1] - at < step ? a.ne[1] - at : step;
+        pa.data = (uint8_t*) a.data + at * (int64_t) a.nb[1];
+        pd.data = (uint8_t*) d.data + at * (int64_t) d.nb[0];
+        const int rc = launch_mul_mat_f32(pa, pb, pd, stream, accumulate);
+        if (rc != TRC_HIP_OK) return rc;
+    }
+    return TRC_HIP_OK;
+}
 
 int launch_mul_mat_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const trc_hip_tensor& d,
                        hipStream_t stream, bool accumulate) {
@@ -616,6 +654,9 @@ int launch_mul_mat_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const t
         s.d_nb0 = p.d_nb0; s.d_nb1 = p.d_nb1; s.d_nb2 = p.d_nb2; s.d_nb3 = p.d_nb3;
         s.accumulate = accumulate ? 1 : 0;
         s.row_blocks = (p.M + 15) / 16;
+        if (s.row_blocks * planes > max_groups(SK_WAVES * 64)) {
+            return mul_mat_in_pieces(a, b, d, s.row_blocks, max_groups(SK_WAVES * 64), stream, accumulate);
+        }
         s.x_span = x_span;
         s.chunks = (int) ((p.K + 31) / 32);
         // K_CONTIG operands are 16-byte aligned with K % 4 == 0; anything else is read element by element
@@ -658,6 +699,9 @@ int launch_mul_mat_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const t
     // error 2.53e-8 here, 2.60e-8 there; from K = 2 on it is smaller there, 3.11e-8
     // against 2.62e-8).
     const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * planes;
+    if (tiles64 > max_groups(256)) {
+        return mul_mat_in_pieces(a, b, d, tiles64 / planes, max_groups(256), stream, accumulate);
+    }
     const int64_t big_tiles = ((p.M + 127) / 128) * ((p.N + 127) / 128) * planes;
     if (p.K > 16 && mm_bf3_fits(p)) {
         // added into dst: K stays in one part
