@@ -324,7 +324,9 @@ __device__ __forceinline__ double sum_chain(double s, const double* p, int n) {
 // or wait lies between. Bound by two launches, then by HBM (65536 x 4096 5.6 TB/s).
 // Chain -> here, both launches: [777, 130] 13.0 -> 6.7 us, [4096, 512] 37.2 -> 6.8,
 // [333, 7992 rows] 68.5 -> 7.5, [4096, 65536] 954 -> 191; where the chain has to run
-// all the same, 4.5 us more.
+// all the same, 4.5 us more, and a fifth more for long 16-byte aligned rows of which there
+// are few (its loop is not unrolled: one row of 100000 555 -> 680; unrolled, 590, but
+// [4096, 4096] with its many workgroups 75 -> 94).
 constexpr int SUMB_THREADS = 1024;
 constexpr int SUMB_MAX = SB_THREADS;  // workgroups: a pair for each thread of the second launch
 constexpr int SUMB_V = 4;             // float4s in flight per thread

@@ -8,12 +8,22 @@
 // the matrix core; the three left out (m l, l m, l l) are under 2^-24 |x y|.
 // Six v_mfma_f32_32x32x16_bf16 take 192 cycles of a SIMD for 32 x 32 x 16
 // products where v_mfma_f32_32x32x2_f32 takes 512 (and runs at the rate of the
-// vector ALU's FMAs). Error against 64 bits is below that of the FP32
-// instructions from K = 2 on (K = 1 does not come here), because a bf16
-// instruction rounds its accumulator once per 16 k: rel 2-norm for normal inputs, FP32 -> here: K = 32
-// 1.05e-7 -> 0.40e-7, 128 1.95e-7 -> 0.64e-7, 1024 5.8e-7 -> 1.9e-7, 4096
-// 1.15e-6 -> 0.40e-6 (positive inputs at K = 4096 1.01e-6 -> 0.35e-6), and the
-// mean error is as near 0 (K = 4096: 2e-8 -> 5e-9 of the result's 2-norm).
+// vector ALU's FMAs). Measured: 4096 x 4096 x 512 89 us, 193 TFLOP/s of F32
+// products, the matrix cores busy 52 % of the cycles (FP32 instructions 138 us).
+//
+// Error against 64 bits: a bf16 instruction rounds its accumulator to nearest once
+// per 16 k, so that the error grows with sqrt(K / 16) and, from K = 2 on, stays below
+// that of the FP32 instructions, which round at every k (K = 1 does not come here). Rel
+// 2-norm, FP32 -> here: normal inputs K = 32 1.05e-7 -> 0.40e-7, 128 1.95e-7 ->
+// 0.64e-7, 1024 5.8e-7 -> 1.9e-7, 4096 1.15e-6 -> 0.40e-6, 262144 9.1e-6 -> 2.3e-6;
+// uniform in [0, 1) K = 4096 8.4e-7 -> 3.0e-7, 16384 1.7e-6 -> 6.0e-7 with a mean of
+// -5e-8, 262144 1.3e-5 -> 1.5e-6. Before it rounds, the instruction drops what lies
+// far enough below its accumulator's last bit, downwards; the products are kept apart
+// by size for that (below). One kind of input fares worse than on the FP32
+// instructions: operands that are all nearly the same number, whose 16-bit first
+// products lose the same bits at every rounding (1 + 0.01 u, K = 4096 8.5e-7 -> 3.4e-7,
+// but 8192 in one chain 1.2e-6 -> 5.6e-6, 65536 4.5e-6 -> 1.8e-5; at 262144 3.2e-4 ->
+// 1.7e-5). A chain is K over the parts, and over two where a tile has 8 waves.
 //
 // Operands are split as x 2^24 and results scaled back by 2^-48, both exact: every
 // part is then 0 or at least 2^-125, a normal bf16, down to the smallest
