@@ -96,19 +96,22 @@ __device__ __forceinline__ void b3_split(float x, float y, uint32_t& h, uint32_t
 // converted. An R_CONTIG quad that holds the operand's last row may hold up to
 // three rows after it, whatever lies there: they reach only sums outside dst.
 // 4-byte alignment is enough for the 16-byte loads.
-template <int MODE, int G>
+// NP: pieces per thread; 1 leaves rows 64 to 127 out (not R_CONTIG), for a tile whose
+// last 64 columns lie past dst.
+template <int MODE, int G, int NP = 2>
 struct B3Slab {
+    static_assert(NP == 2 || MODE != MM_R_CONTIG, "a row-contiguous piece is four rows of one k");
     static constexpr int RS = MODE == MM_R_CONTIG ? 32 * 16 + 32 : 0;
     static constexpr int HS = MODE == MM_R_CONTIG ? 4 * RS : (G == 1 ? 128 * 16 + 128 : 128 * 16 + 64);
     static constexpr int PS = 2 * HS, GS = 3 * PS;
     static constexpr int BYTES = G * GS;
-    uint32_t vo[2];  // byte offset of piece u of slab 0
-    int ko[2];       // its first k within a slab
-    uint32_t lo;     // LDS byte offset of piece 0
+    uint32_t vo[NP];  // byte offset of piece u of slab 0
+    int ko[NP];       // its first k within a slab
+    uint32_t lo;      // LDS byte offset of piece 0
     uint32_t nb0;
-    uint32_t step;   // bytes from one slab to the next
+    uint32_t step;    // bytes from one slab to the next
     __amdgpu_buffer_rsrc_t rs;
-    f4 r[2][2];      // [stage][piece]: slab s waits in stage s % 2
+    f4 r[2][NP];      // [stage][piece]: slab s waits in stage s % 2
 
     static __device__ __forceinline__ uint32_t chunk(int row) {
         if constexpr (MODE == MM_R_CONTIG) return (uint32_t) ((row & 3) * RS + (row >> 2) * 16);
@@ -127,7 +130,7 @@ struct B3Slab {
             const int lane = tid & 63, wave = tid >> 6;
             const int q = 8 * (wave & 3) + (lane & 7), kp = (lane >> 3) & 7, g = wave >> 2;
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
+            for (int u = 0; u < NP; ++u) {
                 ko[u] = 16 * g + 2 * kp + u;
                 vo[u] = 4 * q < rows ? (uint32_t) ((k0 + ko[u]) * nbk + 16 * q) : MM_OUT;
             }
@@ -135,7 +138,7 @@ struct B3Slab {
         } else {
             const int row = tid / (4 * G), kq = tid % (4 * G);
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
+            for (int u = 0; u < NP; ++u) {
                 ko[u] = 4 * kq;
                 vo[u] = row + 64 * u < rows ? (uint32_t) ((row + 64 * u) * nbr + (k0 + ko[u]) * nbk) : MM_OUT;
             }
@@ -160,7 +163,7 @@ struct B3Slab {
     // k past K of the last slab, whose first k is `left` before K, becomes 0
     __device__ __forceinline__ void mask(int st, int left) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < NP; ++u)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (ko[u] + (MODE == MM_R_CONTIG ? 0 : e) >= left) r[st][u][e] = 0.f;
@@ -195,7 +198,7 @@ struct B3Slab {
     static constexpr int LDF = B3_T + 1;
     __device__ __forceinline__ void store_f32(float* l, int tid) const {
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < NP; ++u)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 if constexpr (MODE == MM_R_CONTIG) {
@@ -239,7 +242,8 @@ template <int AMODE, int BMODE, int G, int MEET, bool ACC, int NY>
 __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint8_t* lds) {
     static_assert(!ACC || MEET == B3_ALONE, "parts that meet store or add to a dst of their own");
     using SA = B3Slab<AMODE, G>;
-    using SB = B3Slab<BMODE, G>;
+    constexpr int NPB = NY == 1 && BMODE != MM_R_CONTIG ? 1 : 2;
+    using SB = B3Slab<BMODE, G, NPB>;
     constexpr int BK = 16 * G;
     constexpr int BUF = SA::BYTES + SB::BYTES;
     constexpr int RED = G == 2 ? 4 * 64 * 64 * 4 : 0;  // half of every wave's sums
@@ -284,14 +288,14 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             sa.load(st, kt, nk, u);
-            sb.load(st, kt, nk, u);
+            if (u < NPB) sb.load(st, kt, nk, u);
         }
     };
     auto lstore = [&](int st, uint8_t* l) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             sa.store(st, l, u);
-            sb.store(st, l + SA::BYTES, u);
+            if (u < NPB) sb.store(st, l + SA::BYTES, u);
         }
     };
     auto masked = [&](int st, int kt) {
@@ -310,7 +314,7 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             ahead[st][0][u] = sa.fetch(2 + st, nk, u);
-            ahead[st][1][u] = sb.fetch(2 + st, nk, u);
+            if (u < NPB) ahead[st][1][u] = sb.fetch(2 + st, nk, u);
         }
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
@@ -319,7 +323,7 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             sa.r[st][u] = ahead[st][0][u];
-            sb.r[st][u] = ahead[st][1][u];
+            if (u < NPB) sb.r[st][u] = ahead[st][1][u];
         }
     }
     __syncthreads();
@@ -373,11 +377,13 @@ __device__ __forceinline__ void b3_tile(const MMArgs& p, const B3Place& at, uint
             if (q == 1) fragsA(rd, 2), sa.store(ST, nxt, 0);
             if (q == 2) fragsB(rd, 2), sa.store(ST, nxt, 1);
             if (q == 3) fragsA(rd, 1), sb.store(ST, nxt + SA::BYTES, 0);
-            if (q == 4) fragsB(rd, 1), sb.store(ST, nxt + SA::BYTES, 1);
+            if (q == 4) fragsB(rd, 1);
+            if (q == 4 && NPB == 2) sb.store(ST, nxt + SA::BYTES, NPB - 1);
             if (q == 5) fragsA(rd, 0), fragsB(rd, 0);
             if constexpr (!decltype(last)::value) {
                 if (q == 2) sa.load(ST, kt + 4, nk, 0), sa.load(ST, kt + 4, nk, 1);
-                if (q == 4) sb.load(ST, kt + 4, nk, 0), sb.load(ST, kt + 4, nk, 1);
+                if (q == 4) sb.load(ST, kt + 4, nk, 0);
+                if (q == 4 && NPB == 2) sb.load(ST, kt + 4, nk, NPB - 1);
             }
             // after each MFMA at most two LDS accesses, a load and six vector
             // instructions (left to itself the compiler moves the conversion
