@@ -25,19 +25,25 @@ B3Plan mm_bf3_plan(const MMArgs& p, int64_t planes, int max_parts) {
     // 19 to 24). 4096 x 4096 x 128, parts 1, 2, 3, 4, 6, 8: 107.6, 63.0, 45.5,
     // 38.9, 34.9, 39.2; 1024 x 1024 x 512: 32.3, 25.1, 20.6, 20.9, 21.9, 27.2.
     // Operands that run along neither dimension load element by element, and with
-    // them the other operand: a slab takes 2.4 with one such operand, 3.3 with two,
-    // 0.6 of that where the last 64 columns are empty, and a launch that fills the
-    // chip 12 more (256 x 256 x 512 in two parts 35 and 42, 1408 x 1408 x 1024 60 and
-    // 74, 1408 x 1408 x 512 40 and 47); 3.5 where two workgroups share a CU and src0
-    // is strided (4096 x 4096 x 512 231, with src1 strided 150).
+    // them the other operand: a slab takes 2.4 with one such operand, 3.3 with two
+    // (0.6 of that with up to 64 columns; with up to 64 rows 0.65, or 0.35), and a
+    // launch that fills the chip 12 more, 6 with up to 64 columns (256 x 256 x 512 in
+    // two parts 35 and 42, 1408 x 1408 x 1024 60 and 74, 1408 x 1408 x 512 40 and 47). K
+    // whole, two workgroups to a CU and src0 strided 3.5 for each tile of a CU (4096 x
+    // 4096 x 512 231, with src1 strided 150).
     const int64_t tiles = ((p.M + B3_T - 1) / B3_T) * ((p.N + B3_T - 1) / B3_T) * planes;
     const int64_t cus = device_cus();
     const double slabs = (double) ((p.K + 31) / 32);
     const bool sa = mm_a_strided(p), sb = mm_b_strided(p);
     const bool narrow = p.N <= 64, strided = sa || sb;
-    const double slab = strided ? (sa && sb ? 3.3 : sa && tiles > cus ? 3.5 : 2.4) * (narrow ? 0.6 : 1) : narrow ? 0.7 : 0.8;
-    auto base = [&](int64_t groups) { return strided ? 12 * (groups < cus ? (double) groups / cus : 1.0) : 0; };
-    B3Plan best{2, 1, base(tiles) + 7.5 + slab * slabs * (double) ((tiles + cus - 1) / cus)};
+    const double part_of = p.M <= 64 ? (narrow ? 0.35 : 0.65) : narrow ? 0.6 : 1;
+    const double slab = strided ? (sa && sb ? 3.3 : 2.4) * part_of : narrow ? 0.7 : 0.8;
+    const double slab1 = sa && !sb && tiles > cus ? 3.5 * part_of : slab;
+    auto base = [&](int64_t groups) {
+        return strided ? (narrow ? 6 : 12) * (groups < cus ? (double) groups / cus : 1.0) : 0;
+    };
+    const double rounds = strided && tiles > cus ? (double) tiles / cus : (double) ((tiles + cus - 1) / cus);
+    B3Plan best{2, 1, base(tiles) + 7.5 + slab1 * slabs * rounds};
     for (int parts = 2; parts <= max_parts; ++parts) {
         // a part is at least 4 slabs: shorter ones are all launch and meeting
         if (slabs < 4 * parts || tiles * parts > (parts == 2 ? 4 * cus : cus)) break;

@@ -685,34 +685,38 @@ int launch_mul_mat_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const t
 
     // Tiles of 64 x 64 with the FP32 instructions take 5 us and 0.7 us per 32 k
     // (0.85 to 1.1 us where an operand loads element by element), up to about 400 of
-    // them; where one operand runs along neither dimension 1.06 us, where both do 1.8,
-    // for each 256 of them and at least 1.3 and 2, or 1.6 for up to 64 columns
-    // (3.1 and 4.25 for each 256 tiles of 128 x 128, from 512 of those on: 4096 x 4096 x
-    // 512 205 and 272 us). The bf16 tiles are taken where their model's time is less (measured, FP32 -> bf16: 768 x
-    // 2048 x 256 21.1 -> 19.1, 512 x 512 x 515 unaligned 24.6 -> 16.1; 512 x 512 x
-    // 512 15.1 -> 15.7, 300 x 300 x 300 11.0 -> 14.0; with src0 strided 1024 x 1024 x
-    // 1024 50 -> 41, 1024 x 1024 x 512 24 -> 36).
-    // Up to 16 k always stay here: the bf16 tiles' slab would be half empty (K = 1, 4
-    // and 16, 4096 x 4096: 17.8 us here, 19.4 there; added to dst 25 and 27), and at
-    // K = 1 they round worse: leaving out the smallest partial products costs up to an
-    // ulp where the FP32 instruction's one product is rounded correctly (2-norm of the
-    // error 2.53e-8 here, 2.60e-8 there; from K = 2 on it is smaller there, 3.11e-8
-    // against 2.62e-8).
+    // them; where one operand runs along neither dimension 1.06 us, or 1.8 where the
+    // other loads by element too and not along its rows, for each 256 of them and at
+    // least 1.3 and 2, or 1.6 for up to 64 columns, 1.05 for up to 64 rows (3.1 and 4.25 for each 256 tiles of 128 x 128, from 512 of
+    // those on: 4096 x 4096 x 512 205 and 272 us). The bf16 tiles are taken where their
+    // model's time is less (measured, FP32 -> bf16: 768 x 2048 x 256 21.1 -> 19.1, 512 x
+    // 512 x 515 unaligned 24.6 -> 16.1; 512 x 512 x 512 15.1 -> 15.7, 300 x 300 x 300
+    // 11.0 -> 14.0; with src0 strided 1024 x 1024 x 1024 50 -> 41, 1024 x 1024 x 512
+    // 24 -> 36).
+    // K = 1 always stays here: leaving out the smallest partial products costs the bf16
+    // tiles up to an ulp where the FP32 instruction's one product is rounded correctly
+    // (2-norm of the error 2.53e-8 here, 2.60e-8 there; from K = 2 on it is smaller
+    // there, 3.11e-8 against 2.62e-8). Up to 16 k, whose bf16 slab is half empty, whole
+    // tiles and strided operands too (4096 x 4096 x 4 17.5 us here, 19.4 there, added to
+    // dst 25 and 27; elsewhere the stores decide: 524 x 2996 x 4 in 64 planes 268 and 228).
     const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * planes;
     if (tiles64 > max_groups(256)) {
         return mul_mat_in_pieces(a, b, d, tiles64 / planes, max_groups(256), stream, accumulate);
     }
     const int64_t big_tiles = ((p.M + 127) / 128) * ((p.N + 127) / 128) * planes;
-    if (p.K > 16 && mm_bf3_fits(p)) {
+    const bool strided = mm_a_strided(p) || mm_b_strided(p);
+    const bool fp32 = p.K == 1 || (p.K <= 16 && ((p.M % 128 == 0 && p.N % 128 == 0) || strided));
+    if (!fp32 && mm_bf3_fits(p)) {
         // added into dst: K stays in one part
         const B3Plan plan = mm_bf3_plan(p, planes, accumulate ? 1 : 8);
         const double slabs = (double) ((p.K + 31) / 32);
-        const bool sa = mm_a_strided(p), sb = mm_b_strided(p);
         double slab = (am == GENERIC || bm == GENERIC ? 0.85 : 0.7) * (tiles64 > 400 ? (double) tiles64 / 400 : 1.0);
-        if (sa || sb) {
-            slab = big_tiles >= 512 ? (sa && sb ? 4.25 : 3.1) * (double) ((big_tiles + 255) / 256)
-                   : tiles64 > 256  ? (sa && sb ? 1.8 : 1.06) * (double) ((tiles64 + 255) / 256)
-                                    : (sa && sb ? (p.N > 64 ? 2.0 : 1.6) : 1.3);
+        if (strided) {
+            const bool both = am == GENERIC && p.a_nb1 != 4 && bm == GENERIC && p.b_nb1 != 4;
+            slab = big_tiles >= 512 ? (both ? 4.25 : 3.1) * (double) ((big_tiles + 255) / 256)
+                   : tiles64 > 256  ? (both ? 1.8 : 1.06) * (double) ((tiles64 + 255) / 256)
+                   : p.M <= 64      ? 1.05
+                                    : (both ? (p.N > 64 ? 2.0 : 1.6) : 1.3);
         }
         if (plan.us < 5 + slab * slabs) return launch_mm_bf3(p, planes, plan.groups, plan.parts, accumulate, stream);
     }
