@@ -698,7 +698,7 @@ int launch_mul_mat_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const t
     // (2-norm of the error 2.53e-8 here, 2.60e-8 there; from K = 2 on it is smaller
     // there, 3.11e-8 against 2.62e-8). Up to 16 k, whose bf16 slab is half empty, whole
     // tiles and strided operands too (4096 x 4096 x 4 17.5 us here, 19.4 there, added to
-    // dst 25 and 27; elsewhere the stores decide: 524 x 2996 x 4 in 64 planes 268 and 228).
+    // dst 25 and 27; elsewhere the stores decide: 524 x 2996 x 4 in 64 planes 268 and 236).
     const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * planes;
     if (tiles64 > max_groups(256)) {
         return mul_mat_in_pieces(a, b, d, tiles64 / planes, max_groups(256), stream, accumulate);
