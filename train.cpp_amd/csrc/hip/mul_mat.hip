@@ -522,7 +522,9 @@ __global__ __launch_bounds__(SK_WAVES * 64) void k_mm_skinny(SkArgs p) {
 template <int NT, int AHEAD>
 int launch_skinny_nt(SkArgs& p, int bmode, int64_t planes, hipStream_t stream) {
     const int64_t grid = p.row_blocks * planes;
-    if (grid > max_groups(SK_WAVES * 64)) return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) grid);
+    if (grid > max_groups(SK_WAVES * 64)) {
+        return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) grid);
+    }
     if (NT == 1 && bmode == K_CONTIG && p.N > 4 && p.N <= 8) {
         // 5..8 columns: X in full lines (at 4 or fewer the 16-column loads are as fast)
         hipLaunchKernelGGL((k_mm_skinny<1, AHEAD, SK_X8>), dim3((unsigned) grid), dim3(SK_WAVES * 64), 0, stream, p);
@@ -553,7 +555,9 @@ int launch_cfg(MMArgs& p, int64_t planes, hipStream_t stream) {
     p.tiles_i = (p.M + BM - 1) / BM;
     p.tiles_j = (p.N + BN - 1) / BN;
     const int64_t grid = p.tiles_i * p.tiles_j * planes;
-    if (grid > max_groups(WI * WJ * 64)) return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) grid);
+    if (grid > max_groups(WI * WJ * 64)) {
+        return fail(TRC_HIP_E_SHAPE, "mul_mat: %lld workgroups exceed one launch", (long long) grid);
+    }
     p.xcd_planes = planes % 8 == 0 ? 1 : 0;
     p.d_span = (p.M - 1) * p.d_nb0 + (p.N - 1) * p.d_nb1 + 4;
     hipLaunchKernelGGL((k_mul_mat<WI, WJ, TI, TJ, BK, AM, BMO, ACC>), dim3((unsigned) grid),
@@ -687,12 +691,12 @@ int launch_mul_mat_f32(const trc_hip_tensor& a, const trc_hip_tensor& b, const t
     // (0.85 to 1.1 us where an operand loads element by element), up to about 400 of
     // them; where one operand runs along neither dimension 1.06 us, or 1.8 where the
     // other loads by element too and not along its rows, for each 256 of them and at
-    // least 1.3 and 2, or 1.6 for up to 64 columns, 1.05 for up to 64 rows (3.1 and 4.25 for each 256 tiles of 128 x 128, from 512 of
-    // those on: 4096 x 4096 x 512 205 and 272 us). The bf16 tiles are taken where their
-    // model's time is less (measured, FP32 -> bf16: 768 x 2048 x 256 21.1 -> 19.1, 512 x
-    // 512 x 515 unaligned 24.6 -> 16.1; 512 x 512 x 512 15.1 -> 15.7, 300 x 300 x 300
-    // 11.0 -> 14.0; with src0 strided 1024 x 1024 x 1024 50 -> 41, 1024 x 1024 x 512
-    // 24 -> 36).
+    // least 1.3 and 2, or 1.6 for up to 64 columns, 1.05 for up to 64 rows (3.1 and 4.25
+    // for each 256 tiles of 128 x 128, from 512 of those on: 4096 x 4096 x 512 205 and
+    // 272 us). The bf16 tiles are taken where their model's time is less (measured,
+    // FP32 -> bf16: 768 x 2048 x 256 21.1 -> 19.1, 512 x 512 x 515 unaligned 24.6 ->
+    // 16.1; 512 x 512 x 512 15.1 -> 15.7, 300 x 300 x 300 11.0 -> 14.0; with src0
+    // strided 1024 x 1024 x 1024 50 -> 41, 1024 x 1024 x 512 24 -> 36).
     // K = 1 always stays here: leaving out the smallest partial products costs the bf16
     // tiles up to an ulp where the FP32 instruction's one product is rounded correctly
     // (2-norm of the error 2.53e-8 here, 2.60e-8 there; from K = 2 on it is smaller
